@@ -79,11 +79,9 @@ int ensure_cache(pm_context* c) {
   }
   const uint32_t R = kChunk;
   HIPCHK(k.X.ensure(2ull * R * MLP_KPAD));
-  for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) HIPCHK(k.H[l].ensure(2ull * R * MLP_HID));
+  for (int j = 0; j < 2; ++j) HIPCHK(k.H[j].ensure(2ull * R * MLP_HID));
   HIPCHK(k.y.ensure(4ull * R * MLP_OUTPAD));
-  HIPCHK(k.dy.ensure(2ull * R * MLP_OUTPAD));
   HIPCHK(k.row_err.ensure(4ull * R));
-  k.tb.dy = k.dy.as<uint16_t>();
   k.tb.row_err = k.row_err.as<float>();
   k.rows_cap = R;
   k.ready = true;
@@ -127,25 +125,17 @@ int sync_ema(pm_context* c) {
   return PM_OK;
 }
 
-uint16_t* const* hidden_ptrs(CacheState& k, uint16_t** tmp) {
-  for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) tmp[l] = k.H[l].as<uint16_t>();
-  return tmp;
-}
-
 }  // namespace
 
 namespace pm {
 void cache_release(CacheState& k) {
-  for (DevBuf* b : {&k.params, &k.grads, &k.adam_m, &k.adam_v, &k.params_bf16, &k.params_ema, &k.ema_bf16, &k.X, &k.y, &k.dy,
+  for (DevBuf* b : {&k.params, &k.grads, &k.adam_m, &k.adam_v, &k.params_bf16, &k.params_ema, &k.ema_bf16, &k.X, &k.y, &k.H[0], &k.H[1],
                     &k.row_err, &k.rgb, &k.err_sum, &k.err_cnt, &k.rec_cnt, &k.rec_off, &k.rec_in,
                     &k.rec_wt, &k.rec_code, &k.rec_val, &k.sel_in, &k.sel_t, &k.list, &k.list_cnt, &k.cell_fb,
                     &k.row_code, &k.row_list, &k.loss_part, &k.loss_acc, &k.rec_q, &k.map_hash, &k.list_fb,
                     &k.XT, &k.dT[0], &k.dT[1], &k.dT[2], &k.dT[3], &k.dyT, &k.tpart})
     b->release();
-  for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) {
-    k.H[l].release();
-    k.HT[l].release();
-  }
+  for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) k.HT[l].release();
   k.ready = false;
 }
 
@@ -248,8 +238,6 @@ int cache_train_dev(pm_context* c, const float* in, const float* target, uint32_
   if (r != PM_OK) return r;
   CacheState& k = c->cache;
   if (batch == 0 || batch > kChunk) return PM_ERR_INVALID;
-  uint16_t* tmp[MLP_HIDDEN_LAYERS];
-  uint16_t* const* H = hidden_ptrs(k, tmp);
   MlpTrainT tt;
   if ((r = ensure_train_t(k, batch, tt)) != PM_OK) return r;
   if ((r = sync_ema(c)) != PM_OK) return r;
@@ -267,8 +255,8 @@ int cache_train_dev(pm_context* c, const float* in, const float* target, uint32_
     }
     MlpTrainBufs tb = k.tb;
     tb.row_err = k.row_err.as<float>() + ro;
-    HIPCHK(mlp_train_grads(k.w, in + (size_t)o * MLP_IN, batch, H, k.y.as<float>(),
-                           target + (size_t)o * MLP_OUT, tb, tt, false, c->stream, esum, ecnt));
+    HIPCHK(mlp_train_grads(k.w, in + (size_t)o * MLP_IN, batch, target + (size_t)o * MLP_OUT, tb, tt, false, c->stream,
+                           esum, ecnt));
     k.step += 1;
     HIPCHK(mlp_adam(k.w, tb, lr, k.step, c->stream, &tt));
     ro += batch;
@@ -319,12 +307,9 @@ int pm_cache_grad(pm_context* c, const float* in_dev, const float* target_dev, u
   int r = ensure_cache(c);
   if (r != PM_OK) return r;
   CacheState& k = c->cache;
-  uint16_t* tmp[MLP_HIDDEN_LAYERS];
-  uint16_t* const* H = hidden_ptrs(k, tmp);
   MlpTrainT tt;
   if ((r = ensure_train_t(k, n, tt)) != PM_OK) return r;
-  HIPCHK(mlp_train_grads(k.w, in_dev, n, H, k.y.as<float>(), target_dev, k.tb, tt, true,
-                         c->stream));
+  HIPCHK(mlp_train_grads(k.w, in_dev, n, target_dev, k.tb, tt, true, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(grad_host, k.grads.p, 4ull * count, hipMemcpyDeviceToHost));
   if (loss) {

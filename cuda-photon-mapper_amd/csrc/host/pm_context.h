@@ -54,7 +54,7 @@ struct MapBufs {
 // Learned radiance cache state: parameters, Adam moments, training scratch.
 struct CacheState {
   DevBuf params, grads, adam_m, adam_v, params_bf16, params_ema, ema_bf16;
-  DevBuf X, H[MLP_HIDDEN_LAYERS], y, dy, row_err, rgb;
+  DevBuf X, H[2], y, row_err, rgb;
   DevBuf XT, HT[MLP_HIDDEN_LAYERS], dT[MLP_HIDDEN_LAYERS], dyT, tpart;  // training: transposes and split partials
   MlpDev w;
   MlpTrainBufs tb;

@@ -28,6 +28,23 @@ inline int mlp_kin(int l) { return l == 0 ? MLP_KPAD : MLP_HID; }
 inline int mlp_nout(int l) { return l == MLP_HIDDEN_LAYERS ? MLP_OUTPAD : MLP_HID; }
 inline size_t mlp_w_count(int l) { return (size_t)mlp_nout(l) * (size_t)mlp_kin(l); }
 inline size_t mlp_b_count(int l) { return (size_t)mlp_nout(l); }
+#if defined(__HIPCC__)
+// p[0] + p[stride] + ... over n slices, added in slice order; the loads of 8
+// slices are issued before they are added.
+__device__ __forceinline__ float slice_sum(const float* p, size_t stride, int n) {
+  float s = 0.0f;
+  int z = 0;
+  for (; z + 8 <= n; z += 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = p[(size_t)(z + j) * stride];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += v[j];
+  }
+  for (; z < n; ++z) s += p[(size_t)z * stride];
+  return s;
+}
+#endif
 inline size_t mlp_param_count() {
   size_t n = 0;
   for (int l = 0; l < MLP_LAYERS; ++l) n += mlp_w_count(l) + mlp_b_count(l);
@@ -54,7 +71,6 @@ struct MlpDev {
 };
 
 struct MlpTrainBufs {
-  uint16_t* dy;       // [rows x OUTPAD]
   float* row_err;     // [rows]
   float* gw[MLP_LAYERS];
   float* gb[MLP_LAYERS];
@@ -79,16 +95,15 @@ struct MlpTrainT {
 int mlp_train_slices(uint32_t rows);
 uint32_t mlp_train_ld(uint32_t rows);
 size_t mlp_train_partial_floats(uint32_t rows);
-// Encode, forward (keeping H and its transposes), loss, backward for `rows`
-// inputs / targets: y the outputs, tb.row_err the per-row squared errors, and
-// the gradients as split partials (tt.part_w / part_b); with `reduce` they are
-// also summed into tb.gw / tb.gb (mlp_adam can instead sum them itself).
+// Encode, forward, loss, backward for `rows` inputs / targets: tb.row_err the
+// per-row squared errors, and the gradients as split partials (tt.part_w /
+// part_b); with `reduce` they are also summed into tb.gw / tb.gb (mlp_adam can instead sum them itself).
 // With esum / ecnt, each row's squared error (capped at 1e6, in 2^-24 fixed
 // point) is also added to the error tracker's cell of its input (err_cell),
 // and the cell's row count incremented.
-hipError_t mlp_train_grads(const MlpDev& w, const float* in, uint32_t rows, uint16_t* const* H,
-                           float* y, const float* target, MlpTrainBufs& tb, MlpTrainT& tt, bool reduce,
-                           hipStream_t st, unsigned long long* esum = nullptr, unsigned int* ecnt = nullptr);
+hipError_t mlp_train_grads(const MlpDev& w, const float* in, uint32_t rows, const float* target, MlpTrainBufs& tb,
+                           MlpTrainT& tt, bool reduce, hipStream_t st, unsigned long long* esum = nullptr,
+                           unsigned int* ecnt = nullptr);
 
 hipError_t mlp_encode(const float* in, uint32_t n, uint16_t* out, hipStream_t st);
 hipError_t mlp_forward(const MlpDev& w, const uint16_t* X, uint32_t rows, uint16_t* const* H, float* y,

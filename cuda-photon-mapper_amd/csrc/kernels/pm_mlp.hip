@@ -209,8 +209,7 @@ __global__ void k_adam_all(AdamSegs S, float lr, float b1, float b2, float eps, 
   float* v = S.v[s];
   float gr;
   if (S.slices > 0) {  // the same fixed-order sum over slices as k_grad_sum
-    gr = 0.0f;
-    for (int z = 0; z < S.slices; ++z) gr += S.gp[s][(size_t)z * S.n[s] + i];
+    gr = slice_sum(S.gp[s] + i, S.n[s], S.slices);
   } else {
     gr = S.g[s][i];
   }

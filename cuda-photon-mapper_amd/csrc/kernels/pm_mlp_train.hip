@@ -1,7 +1,7 @@
-// pm_mlp_train.hip -- the learned cache's training pass (forward with stored
-// activations, backward, weight and bias gradients) on gfx950: the forward
-// pass and loss gradient in one fused kernel (k_fwd_fused), the backward
-// products on one "NT" GEMM kernel whose operands are both contiguous along K.
+// pm_mlp_train.hip -- the learned cache's training pass (forward, loss,
+// backward, weight and bias gradients) on gfx950, three launches a step with
+// Adam: k_fwd_bwd takes 64 rows through all layers and back with the
+// activations in LDS, k_wgrad computes the five layers' weight gradients.
 //
 // No reference counterpart (the reference has no learned component).
 //
@@ -10,13 +10,13 @@
 //   forward      H_l [rows x out] = X_{l} [rows x in] . W_l [out x in]^T
 //   delta        D_{l-1} [rows x in] = D_l [rows x out] . (W_l^T) [in x out]^T
 //   weight grad  dW_l [out x in] = (D_l^T) [out x rows] . (X_l^T) [in x rows]^T
-// so the forward and delta products also write their output transposed (the
-// weight gradients' operands), the encoder writes X and X^T, and the BF16
-// weights are kept in both orders (W and W^T, refreshed by Adam).  A
-// 256-thread workgroup computes a 64 x 64 tile of C; each wave a 32 x 32
-// quarter on v_mfma_f32_16x16x32_bf16.  K is staged through LDS 128 at a time
-// with 16-byte loads and 16-byte LDS fragment reads.  The weight gradients
-// split the batch (K) over grid.z slices that write FP32 partial tiles, and
+// so k_fwd_bwd writes the encoded inputs, the activations and the deltas
+// transposed (the weight gradients' operands), and the BF16 weights are kept
+// in both orders (W and W^T, refreshed by Adam).  Every element of a product
+// accumulates its K in ascending steps of 32 from zero on
+// v_mfma_f32_16x16x32_bf16, then bias, ReLU or mask, then BF16: which wave
+// computes it, and in which tile, does not change its bits.  The weight
+// gradients split the batch (K) over slices that write FP32 partial tiles, and
 // the bias gradients (row sums of D^T) likewise; the slices of every layer are
 // added in slice order (deterministic), by one kernel or by Adam itself.
 #include "pm_kernels.h"
@@ -27,542 +27,406 @@ namespace pm {
 
 namespace {
 
+// Barrier for data exchanged through LDS only: it does not wait for the
+// wave's global loads and stores, which no other wave of the workgroup reads.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int NT_TILE = 64;  // tile M and N
-constexpr int NT_KC = 128;   // K per LDS stage
-constexpr int NT_LDS = NT_KC + 8;  // LDS row length (bf16), padded
-
-__device__ __forceinline__ float bf_to_f(uint16_t h) { return bf16_to_f32(h); }
-
-struct NtArgs {
-  int M, N, K;
-  const uint16_t* A;  // A[m * lda + k]
-  int lda;
-  const uint16_t* B;  // B[n * ldb + k]
-  int ldb;
-  // epilogue of an unsplit product
-  const float* bias;       // + bias[n]
-  int relu;                // max(0, .)
-  const uint16_t* mask;    // * (mask[m * ldm + n] > 0)
-  int ldm;
-  uint16_t* Cb;            // BF16 C[m * ldc + n]
-  int ldc;
-  uint16_t* Ct;            // BF16 C^T[n * ldt + m] (ldt >= M rounded up to 64)
-  int ldt;
-  float* Cf;               // FP32 C[m * ldf + n]
-  int ldf;
-  // split product (gridDim.z slices of kps): partial tiles part[z][m][n],
-  // and when bpart is set the row sums of A over the slice, bpart[z][m]
-  int kps;
-  float* part;
-  float* bpart;
-};
-
-// Stages A rows [m0, m0+64) and B rows [n0, n0+64), k in [k0, k0 + kc) (kc a
-// multiple of 32), into LDS; elements outside M, N or k_end are zero.
-__device__ __forceinline__ void nt_stage(const NtArgs& g, uint16_t (*As)[NT_LDS], uint16_t (*Bs)[NT_LDS], int m0,
-                                         int n0, int k0, int kc, int k_end) {
-  const int vec_per_row = kc / 8;
-  for (int v = (int)threadIdx.x; v < 2 * NT_TILE * vec_per_row; v += 256) {
-    const bool isB = v >= NT_TILE * vec_per_row;
-    const int w = isB ? v - NT_TILE * vec_per_row : v;
-    const int r = w / vec_per_row, kk = (w % vec_per_row) * 8;
-    const int gr = (isB ? n0 : m0) + r, gk = k0 + kk;
-    const int rlim = isB ? g.N : g.M;
-    const uint16_t* src = isB ? g.B + (size_t)gr * g.ldb + gk : g.A + (size_t)gr * g.lda + gk;
-    uint4 q = make_uint4(0u, 0u, 0u, 0u);
-    if (gr < rlim) {
-      if (gk + 8 <= k_end) {
-        q = *(const uint4*)src;
-      } else if (gk < k_end) {
-        uint16_t e[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) e[j] = gk + j < k_end ? src[j] : (uint16_t)0;
-        q.x = (uint32_t)e[0] | ((uint32_t)e[1] << 16);
-        q.y = (uint32_t)e[2] | ((uint32_t)e[3] << 16);
-        q.z = (uint32_t)e[4] | ((uint32_t)e[5] << 16);
-        q.w = (uint32_t)e[6] | ((uint32_t)e[7] << 16);
-      }
-    }
-    uint16_t* dst = isB ? &Bs[r][kk] : &As[r][kk];
-    *(uint4*)dst = q;
-  }
-}
-
-// Tile (bx, by) of slice bz (of nz) of the product g.
-__device__ __forceinline__ void nt_tile(const NtArgs& g, int bx, int by, int bz, int nz, uint16_t (*As)[NT_LDS],
-                                        uint16_t (*Bs)[NT_LDS]) {
-  const int lane = lane_id();
-  const int wave = (int)(threadIdx.x >> 6);
-  const int m0 = by * NT_TILE, n0 = bx * NT_TILE;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const bool split = nz > 1 || g.part;
-  const int k_begin = split ? bz * g.kps : 0;
-  const int k_end = split ? min(g.K, k_begin + g.kps) : g.K;
-  const int r16 = lane & 15, q = lane >> 4;
-  f32x4_t acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  float rowsum = 0.0f;  // bias gradient: row threadIdx.x of A over this slice (n-tile 0)
-  const bool want_rowsum = g.bpart && bx == 0 && threadIdx.x < NT_TILE;
-  // the epilogue's bias and mask values, loaded before the K loop so that
-  // their latency overlaps the operand loads
-  float bias_v[2] = {0.0f, 0.0f};
-  uint16_t mask_v[2][2][4];
-  if (!split) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int n = n0 + wn + 16 * b + r16;
-      if (g.bias && n < g.N) bias_v[b] = g.bias[n];
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int m = m0 + wm + 16 * a + 4 * q + e, n = n0 + wn + 16 * b + r16;
-          // 0x3f80 is 1.0 in BF16: kept when there is no mask
-          mask_v[a][b][e] = g.mask && m < g.M && n < g.N ? g.mask[(size_t)m * g.ldm + n] : (uint16_t)0x3f80;
-        }
-  }
-  for (int k0 = k_begin; k0 < k_end; k0 += NT_KC) {
-    const int kc = min(NT_KC, (k_end - k0 + 31) / 32 * 32);
-    nt_stage(g, As, Bs, m0, n0, k0, kc, k_end);
-    __syncthreads();
-    if (want_rowsum)
-      for (int k = 0; k < kc; ++k) rowsum += bf_to_f(As[threadIdx.x][k]);
-    for (int ks = 0; ks < kc; ks += 32) {
-      bf16x8_t af[2], bfr[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const uint4 va = *(const uint4*)&As[wm + t * 16 + r16][ks + 8 * q];
-        af[t] = *(const bf16x8_t*)&va;
-        const uint4 vb = *(const uint4*)&Bs[wn + t * 16 + r16][ks + 8 * q];
-        bfr[t] = *(const bf16x8_t*)&vb;
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // lane holds C[wm + 16a + 4q + e][wn + 16b + r16]
-  if (split) {
-    float* P = g.part + (size_t)bz * g.M * g.N;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int m = m0 + wm + 16 * a + 4 * q + e, n = n0 + wn + 16 * b + r16;
-          if (m < g.M && n < g.N) P[(size_t)m * g.N + n] = acc[a][b][e];
-        }
-    if (want_rowsum && m0 + (int)threadIdx.x < g.M)
-      g.bpart[(size_t)bz * g.M + m0 + threadIdx.x] = rowsum;
-    return;
-  }
-  // unsplit: bias, ReLU, mask, then the BF16 / FP32 outputs; the transposed
-  // BF16 output goes through LDS so its rows are written 16 bytes at a time
-  uint16_t (*T)[NT_TILE + 8] = (uint16_t (*)[NT_TILE + 8])&As[0][0];  // [n][m], 9.2 KB of As
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int ml = wm + 16 * a + 4 * q + e, nl = wn + 16 * b + r16;
-        const int m = m0 + ml, n = n0 + nl;
-        float v = acc[a][b][e];
-        if (n < g.N) {
-          if (g.bias) v += bias_v[b];
-          if (g.relu) v = v > 0.0f ? v : 0.0f;
-          if (!(bf_to_f(mask_v[a][b][e]) > 0.0f)) v = 0.0f;
-        }
-        const uint16_t h = f32_to_bf16(v);
-        if (m < g.M && n < g.N) {
-          if (g.Cb) g.Cb[(size_t)m * g.ldc + n] = h;
-          if (g.Cf) g.Cf[(size_t)m * g.ldf + n] = v;
-        }
-        if (g.Ct) T[nl][ml] = h;
-      }
-  if (g.Ct) {
-    __syncthreads();
-    // 64 rows (n) x 8 vectors of 8 m; columns m >= M land in the padding of C^T
-    for (int v = (int)threadIdx.x; v < NT_TILE * 8; v += 256) {
-      const int nl = v >> 3, j = (v & 7) * 8;
-      if (n0 + nl < g.N) *(uint4*)&g.Ct[(size_t)(n0 + nl) * g.ldt + m0 + j] = *(const uint4*)&T[nl][j];
-    }
-  }
-}
-
-__global__ void __launch_bounds__(256) k_gemm_nt(NtArgs g) {
-  __shared__ __align__(16) uint16_t As[NT_TILE][NT_LDS];
-  __shared__ __align__(16) uint16_t Bs[NT_TILE][NT_LDS];
-  nt_tile(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, As, Bs);
-}
-
-// Independent products in one launch (the five weight gradients of a batch):
-// workgroups [first[s], first[s + 1]) take product s, n-tiles fastest, then
-// m-tiles, then slices.
-struct NtMulti {
-  NtArgs a[MLP_LAYERS];
-  int nx[MLP_LAYERS], ny[MLP_LAYERS], nz[MLP_LAYERS];
-  int first[MLP_LAYERS + 1];
-};
-
-template <int S>
-__device__ __forceinline__ void nt_multi_tile(const NtMulti& p, int c, uint16_t (*As)[NT_LDS], uint16_t (*Bs)[NT_LDS]) {
-  nt_tile(p.a[S], c % p.nx[S], (c / p.nx[S]) % p.ny[S], c / (p.nx[S] * p.ny[S]), p.nz[S], As, Bs);
-}
-
-__global__ void __launch_bounds__(256) k_gemm_nt_multi(NtMulti p) {
-  __shared__ __align__(16) uint16_t As[NT_TILE][NT_LDS];
-  __shared__ __align__(16) uint16_t Bs[NT_TILE][NT_LDS];
-  const int b = (int)blockIdx.x;
-  int s = 0;
-  while (s + 1 < MLP_LAYERS && b >= p.first[s + 1]) ++s;
-  const int c = b - p.first[s];
-  static_assert(MLP_LAYERS == 5, "one case per layer");
-  switch (s) {
-    case 0: nt_multi_tile<0>(p, c, As, Bs); break;
-    case 1: nt_multi_tile<1>(p, c, As, Bs); break;
-    case 2: nt_multi_tile<2>(p, c, As, Bs); break;
-    case 3: nt_multi_tile<3>(p, c, As, Bs); break;
-    default: nt_multi_tile<4>(p, c, As, Bs); break;
-  }
-}
-
-hipError_t gemm_nt(const NtArgs& a, int slices, hipStream_t st) {
-  dim3 grid((unsigned)((a.N + NT_TILE - 1) / NT_TILE), (unsigned)((a.M + NT_TILE - 1) / NT_TILE), (unsigned)slices);
-  hipLaunchKernelGGL(k_gemm_nt, grid, dim3(256), 0, st, a);
-  return hipGetLastError();
-}
-
-// The products g[0..MLP_LAYERS) with slices[s] K slices each, one launch.
-hipError_t gemm_nt_multi(const NtArgs* g, const int* slices, hipStream_t st) {
-  NtMulti p;
-  p.first[0] = 0;
-  for (int i = 0; i < MLP_LAYERS; ++i) {
-    p.a[i] = g[i];
-    p.nx[i] = (g[i].N + NT_TILE - 1) / NT_TILE;
-    p.ny[i] = (g[i].M + NT_TILE - 1) / NT_TILE;
-    p.nz[i] = slices[i];
-    p.first[i + 1] = p.first[i] + p.nx[i] * p.ny[i] * p.nz[i];
-  }
-  hipLaunchKernelGGL(k_gemm_nt_multi, dim3((unsigned)p.first[MLP_LAYERS]), dim3(256), 0, st, p);
-  return hipGetLastError();
-}
-
-NtArgs nt_args(int M, int N, int K) {
-  NtArgs a;
-  memset(&a, 0, sizeof(a));
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  return a;
-}
-
-// ---------------------------------------------------------------- fused forward
-// The forward pass of a training batch in one launch: a workgroup takes 64
-// rows through the five layers with the activations in LDS, writes each
-// hidden layer's output row-major (H_l) and transposed (H_l^T), then the
-// output layer's y and the loss gradient: with t = log(1 + max(target, 0)),
-// d = y - t per channel, dy = 2 d / (3 rows) (BF16, also transposed; zero in
-// the padding columns) and row_err = sum of d^2.  When esum is set, each
-// row's row_err (capped at 1e6) is added in 2^-24 fixed point to the error
-// tracker's cell of its input, and the cell's count incremented (integer
-// atomics: the bins do not depend on the order).  Every
-// product is k_gemm_nt's (the same MFMA operands, K in ascending steps of 32
-// from a zero accumulator, then bias, ReLU and BF16 rounding), so the outputs
-// equal those of one launch per layer bit for bit.  A wave computes the
-// tile's 64 rows x 32 of a hidden layer's 128 outputs, or 16 rows of the 16
-// output-layer columns.
+// ---------------------------------------------------------------- forward and backward
+// A training batch from the inputs to the deltas in one launch.  A workgroup
+// of 16 waves takes 64 rows: it encodes them, runs the five layers, forms the
+// loss gradient (with t = log(1 + max(target, 0)), d = y - t per channel,
+// dy = 2 d / (3 rows), row_err = sum of d^2) and takes it back through the
+// hidden layers, D_{l-1} = (D_l . W_l) x [H_{l-1} > 0].  When esum is set,
+// each row's row_err (capped at 1e6) is added in 2^-24 fixed point to the
+// error tracker's cell of its input, and the cell's count incremented (integer
+// atomics: the bins do not depend on the order).
+//
+// A batch is 128 to 256 workgroups of one per CU, so the time is the chain of
+// nine dependent products of one tile, and what bounds it is latency: the
+// next product's weights are loaded into registers before a product's K loop
+// and written to the other LDS buffer after it (one barrier a product), the
+// ReLU masks stay in registers as one bit per element (the deltas have the
+// activations' shape and lane mapping), and an element's four consecutive
+// rows are stored to the transposed arrays from registers, 8 bytes at a time.
+// Wave w computes n-tile w % 8 of m-tiles 2 (w / 8) and 2 (w / 8) + 1.
+// Two kernels of 4 waves (forward; backward with H, y and dy through memory)
+// took 38 + 32 us for 8,192 rows and 138 + 115 us for 65,536; this one 39 us
+// for 16,384.
 constexpr int FF_XS = MLP_KPAD + 8;  // LDS row length (bf16) of X and W1
-constexpr int FF_HS = MLP_HID + 8;   // of the hidden activations and W2..W5
-constexpr size_t FF_LDS = 2u * (64u * FF_XS + 2u * 64u * FF_HS + 128u * FF_XS) + 4u * 64u * MLP_OUTPAD;
+constexpr int FF_HS = MLP_HID + 8;   // of the hidden activations, deltas and W2..W5
+constexpr int FB_THREADS = 1024;
+constexpr int FB_YS = 4;             // LDS row length (floats) of y and of the targets
+constexpr size_t FB_LDS = 2u * (64u * FF_XS + 2u * 64u * FF_HS + 128u * FF_XS + 128u * FF_HS) + 4u * 2u * 64u * FB_YS;
+static_assert(FB_LDS <= 160u * 1024u, "one workgroup's LDS");
 
-struct FwdArgs {
-  uint16_t* XT;       // [KPAD x ld] encoded inputs, transposed (written here)
+// Two FP32 values to BF16, round to nearest even (one instruction; the bits of
+// f32_to_bf16 for finite values).
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t v = __builtin_convertvector((f32x2_t{a, b}), bf16x2_t);
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+struct FwdBwdArgs {
   uint32_t rows;
-  const uint16_t* w[MLP_LAYERS];
-  const float* b[MLP_LAYERS];
-  uint16_t* H[MLP_HIDDEN_LAYERS];   // [rows x HID]
-  uint16_t* HT[MLP_HIDDEN_LAYERS];  // [HID x ld]
   uint32_t ld;
-  float* y;                         // [rows x OUTPAD]
-  const float* target;              // [rows x OUT]
-  uint16_t* dy;                     // [rows x OUTPAD]
-  uint16_t* dyT;                    // [OUTPAD x ld]
-  float* row_err;                   // [rows]
-  const float* in;                  // [rows x IN] query rows
-  unsigned long long* esum;         // error tracker (null: none)
+  const float* in;                       // [rows x IN] query rows
+  const float* target;                   // [rows x OUT]
+  const uint16_t* w[MLP_LAYERS];
+  const uint16_t* wbt[MLP_LAYERS];       // W_l^T [kin x nout]
+  const float* b[MLP_LAYERS];
+  uint16_t* XT;                          // [KPAD x ld] encoded inputs, transposed
+  uint16_t* HT[MLP_HIDDEN_LAYERS];       // [HID x ld]
+  uint16_t* dT[MLP_HIDDEN_LAYERS];       // [HID x ld]
+  uint16_t* dyT;                         // [OUTPAD x ld]
+  float* row_err;                        // [rows]
+  unsigned long long* esum;              // error tracker (null: none)
   unsigned int* ecnt;
 };
 
-__global__ void __launch_bounds__(256) k_fwd_fused(FwdArgs A) {
+// Weights of one product, on their way from memory to LDS through registers:
+// `nrow` rows of `ncol` (a multiple of 8) at src, row length `ls` in LDS.
+struct WStage {
+  uint4 v[2];
+  __device__ __forceinline__ void load(const uint16_t* src, int nrow, int ncol) {
+    const int per = ncol / 8;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = (int)threadIdx.x + j * FB_THREADS;
+      if (i < nrow * per) v[j] = *(const uint4*)&src[(size_t)i * 8];
+    }
+  }
+  __device__ __forceinline__ void store(uint16_t* dst, int nrow, int ncol) const {
+    const int per = ncol / 8;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = (int)threadIdx.x + j * FB_THREADS;
+      if (i < nrow * per) *(uint4*)&dst[(i / per) * FF_HS + (i % per) * 8] = v[j];
+    }
+  }
+};
+
+// This wave's two 16x16 tiles of act . Ws^T over K = kin.
+__device__ __forceinline__ void fb_product(const uint16_t* act, int as, const uint16_t* Ws, int ws, int kin, int wave,
+                                           int r16, int q, f32x4_t acc[2]) {
+  acc[0] = acc[1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const uint16_t* a0 = &act[(32 * (wave >> 3) + r16) * as + 8 * q];
+  const uint16_t* b0 = &Ws[(16 * (wave & 7) + r16) * ws + 8 * q];
+  for (int ks = 0; ks < kin; ks += 32) {
+    const uint4 va0 = *(const uint4*)&a0[ks], va1 = *(const uint4*)&a0[16 * as + ks], vb = *(const uint4*)&b0[ks];
+    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&va0, *(const bf16x8_t*)&vb, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&va1, *(const bf16x8_t*)&vb, acc[1], 0, 0, 0);
+  }
+}
+
+// Stores the wave's elements h (rows 16 t + 4 q + 0..3 of column n, in pairs)
+// to the LDS tile and, as 8-byte groups, to the transposed array.
+__device__ __forceinline__ void fb_store(const uint32_t h[2][2], uint16_t* out, uint16_t* T, uint32_t ld, uint32_t m0,
+                                         int wave, int r16, int q) {
+  const int n = 16 * (wave & 7) + r16;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int m = 32 * (wave >> 3) + 16 * t + 4 * q;
+    if (out) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[(m + e) * FF_HS + n] = (uint16_t)(h[t][e >> 1] >> (16 * (e & 1)));
+    }
+    *(uint2*)&T[(size_t)n * ld + m0 + (uint32_t)m] = make_uint2(h[t][0], h[t][1]);
+  }
+}
+
+__global__ void __launch_bounds__(FB_THREADS) k_fwd_bwd(FwdBwdArgs A) {
   extern __shared__ __align__(16) unsigned char fl[];
-  uint16_t* Xs = (uint16_t*)fl;                  // [64][FF_XS]
-  uint16_t* Hs[2] = {Xs + 64 * FF_XS, Xs + 64 * FF_XS + 64 * FF_HS};  // [64][FF_HS] each
-  uint16_t* Ws = Xs + 64 * FF_XS + 2 * 64 * FF_HS;  // [128][FF_XS] or [nout][FF_HS]
-  float* ys = (float*)(Ws + 128 * FF_XS);        // [64][OUTPAD]
+  uint16_t* const Xs = (uint16_t*)fl;               // [64][FF_XS]
+  uint16_t* const Hs0 = Xs + 64 * FF_XS;            // [64][FF_HS] each, ping-pong
+  uint16_t* const Hs1 = Hs0 + 64 * FF_HS;
+  uint16_t* const WA = Hs1 + 64 * FF_HS;            // [128][FF_XS]
+  uint16_t* const WB = WA + 128 * FF_XS;            // [128][FF_HS]
+  float* const ys = (float*)(WB + 128 * FF_HS);     // [64][FB_YS] the outputs
+  float* const ts = ys + 64 * FB_YS;                // [64][FB_YS] log(1 + max(target, 0))
   const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6, r16 = lane & 15, q = lane >> 4;
-  const uint32_t m0 = blockIdx.x * 64u;
-  const uint32_t rows = A.rows;
-  // the tile's encoded inputs: {sin, cos}(2 pi 2^(b-1) v) of each input v
-  // at column 24 i + 2b (+1), padding columns and rows past the batch zero
-  for (int v = tid; v < 64 * MLP_IN; v += 256) {
-    const int r = v / MLP_IN, i = v % MLP_IN;
-    const bool ok = m0 + (uint32_t)r < rows;
-    const float x = ok ? A.in[(size_t)(m0 + r) * MLP_IN + i] : 0.0f;
-    uint16_t* o = &Xs[r * FF_XS + i * 2 * MLP_BANDS];
-    float scale = 0.5f;
-    for (int b = 0; b < MLP_BANDS; ++b) {
+  const uint32_t m0 = blockIdx.x * 64u, rows = A.rows;
+  const bool ok = m0 + (uint32_t)lane < rows;       // this lane's row, where a wave's lanes are the rows
+  const float* const in = A.in + (size_t)(m0 + (uint32_t)lane) * MLP_IN;
+  uint4 w0[4];  // W1 on its way to LDS
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int v = tid + j * FB_THREADS;
+    if (v < MLP_HID * (MLP_KPAD / 8)) w0[j] = *(const uint4*)&A.w[0][(size_t)v * 8];
+  }
+  // the tile's encoded inputs: {sin, cos}(2 pi 2^(b-1) v) of each input v at
+  // column 24 i + 2b (+1), padding columns and rows past the batch zero; a
+  // wave takes four bands of an input of the 64 rows at a time
+  for (int i = wave; i < MLP_IN * 3; i += FB_THREADS / 64) {
+    const int v = i / 3, b0 = 4 * (i % 3);
+    uint16_t* xt = A.XT + (size_t)(v * 2 * MLP_BANDS) * A.ld + m0 + (uint32_t)lane;
+    const float x = ok ? in[v] : 0.0f;
+    float scale = 0.5f * (float)(1 << b0);
+#pragma unroll
+    for (int b = b0; b < b0 + 4; ++b) {
       float sn, cs;
       sincos_turns(x * scale, &sn, &cs);
-      o[2 * b] = ok ? f32_to_bf16(sn) : (uint16_t)0;
-      o[2 * b + 1] = ok ? f32_to_bf16(cs) : (uint16_t)0;
+      const uint32_t p = ok ? bf16_pair(sn, cs) : 0u;
+      *(uint32_t*)&Xs[lane * FF_XS + v * 2 * MLP_BANDS + 2 * b] = p;
+      xt[(size_t)(2 * b) * A.ld] = (uint16_t)p;
+      xt[(size_t)(2 * b + 1) * A.ld] = (uint16_t)(p >> 16);
       scale *= 2.0f;
     }
-    if (i == MLP_IN - 1)
-      for (int k = MLP_FEAT; k < MLP_KPAD; ++k) Xs[r * FF_XS + k] = 0;
   }
-  __syncthreads();
-  // X^T: 64 columns of each of its KPAD rows
-  for (int v = tid; v < MLP_KPAD * 8; v += 256) {
-    const int f = v >> 3, j = (v & 7) * 8;
-    uint32_t p[4];
+  // the waves with one encoding task fewer: the targets, the zero rows of X^T
+  // and dy^T, and the rows' error cells
+  uint32_t cell = 0u;
+  if (wave >= 11 && wave < 11 + MLP_OUT) {
+    const int c = wave - 11;
+    ts[lane * FB_YS + c] = ok ? log_(1.0f + fmax_(A.target[(size_t)(m0 + (uint32_t)lane) * MLP_OUT + c], 0.0f)) : 0.0f;
+  } else if (wave == 14) {
+    uint16_t* xt = A.XT + (size_t)MLP_FEAT * A.ld + m0 + (uint32_t)lane;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      p[t] = (uint32_t)Xs[(j + 2 * t) * FF_XS + f] | ((uint32_t)Xs[(j + 2 * t + 1) * FF_XS + f] << 16);
-    *(uint4*)&A.XT[(size_t)f * A.ld + m0 + j] = make_uint4(p[0], p[1], p[2], p[3]);
+    for (int k = 0; k < MLP_KPAD - MLP_FEAT; ++k) xt[(size_t)k * A.ld] = 0;
+    *(uint4*)&Xs[lane * FF_XS + MLP_FEAT] = make_uint4(0u, 0u, 0u, 0u);
+  } else if (wave == 15) {
+    for (int c = MLP_OUT; c < MLP_OUTPAD; ++c)
+      if (ok) A.dyT[(size_t)c * A.ld + m0 + (uint32_t)lane] = 0;
+    if (ok && A.esum) cell = err_cell(in);
   }
-  const uint16_t* act = Xs;
-  int as = FF_XS, kin = MLP_KPAD;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int v = tid + j * FB_THREADS;
+    if (v < MLP_HID * (MLP_KPAD / 8)) *(uint4*)&WA[(v / (MLP_KPAD / 8)) * FF_XS + (v % (MLP_KPAD / 8)) * 8] = w0[j];
+  }
+  lds_barrier();
+  // ---- forward: hidden layers, the weights alternately in WA and WB
+  WStage ww;
+  uint32_t mask = 0u;  // bit 8 l + 4 t + e: element (t, e) of H_l is positive
+  f32x4_t acc[2];
+  uint32_t h[2][2];
+  const int n = 16 * (wave & 7) + r16;
+#pragma unroll
   for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) {
-    const int ws = l == 0 ? FF_XS : FF_HS;
-    __syncthreads();  // the previous layer is done with Ws (and its output tile is complete)
-    for (int v = tid; v < MLP_HID * (kin / 8); v += 256) {
-      const int r = v / (kin / 8), kk = (v % (kin / 8)) * 8;
-      *(uint4*)&Ws[r * ws + kk] = *(const uint4*)&A.w[l][(size_t)r * kin + kk];
-    }
-    __syncthreads();
-    f32x4_t acc[4][2];
+    const int nnext = l + 1 < MLP_HIDDEN_LAYERS ? MLP_HID : MLP_OUTPAD;
+    ww.load(A.w[l + 1], nnext, MLP_HID);
+    const float bias = A.b[l][n];
+    const uint16_t* act = l == 0 ? Xs : ((l & 1) ? Hs0 : Hs1);
+    fb_product(act, l == 0 ? FF_XS : FF_HS, (l & 1) ? WB : WA, l == 0 ? FF_XS : FF_HS, l == 0 ? MLP_KPAD : MLP_HID,
+               wave, r16, q, acc);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int ks = 0; ks < kin; ks += 32) {
-      bf16x8_t af[4], bfr[2];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const uint4 v = *(const uint4*)&act[(16 * a + r16) * as + ks + 8 * q];
-        af[a] = *(const bf16x8_t*)&v;
+      for (int e = 0; e < 4; e += 2) {
+        float v0 = acc[t][e] + bias, v1 = acc[t][e + 1] + bias;
+        v0 = v0 > 0.0f ? v0 : 0.0f;
+        v1 = v1 > 0.0f ? v1 : 0.0f;
+        const uint32_t p = bf16_pair(v0, v1);
+        h[t][e >> 1] = p;
+        mask |= (p & 0xffffu) != 0u ? 1u << (8 * l + 4 * t + e) : 0u;
+        mask |= p >= 0x10000u ? 2u << (8 * l + 4 * t + e) : 0u;
       }
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const uint4 v = *(const uint4*)&Ws[(32 * wave + 16 * b + r16) * ws + ks + 8 * q];
-        bfr[b] = *(const bf16x8_t*)&v;
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
-    }
-    // lane holds C[16a + 4q + e][32 wave + 16b + r16]
-    uint16_t* out = Hs[l & 1];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int n = 32 * wave + 16 * b + r16;
-      const float bias = A.b[l][n];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float v = acc[a][b][e] + bias;
-          v = v > 0.0f ? v : 0.0f;
-          out[(16 * a + 4 * q + e) * FF_HS + n] = f32_to_bf16(v);
-        }
-    }
-    __syncthreads();
-    // H_l rows of the batch, and H_l^T (64 columns of each of its 128 rows)
-    for (int v = tid; v < 64 * (MLP_HID / 8); v += 256) {
-      const int r = v / (MLP_HID / 8), j = (v % (MLP_HID / 8)) * 8;
-      if (m0 + (uint32_t)r < rows) *(uint4*)&A.H[l][(size_t)(m0 + r) * MLP_HID + j] = *(const uint4*)&out[r * FF_HS + j];
-    }
-    for (int v = tid; v < MLP_HID * 8; v += 256) {
-      const int n = v >> 3, j = (v & 7) * 8;
-      uint32_t p[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        p[t] = (uint32_t)out[(j + 2 * t) * FF_HS + n] | ((uint32_t)out[(j + 2 * t + 1) * FF_HS + n] << 16);
-      *(uint4*)&A.HT[l][(size_t)n * A.ld + m0 + j] = make_uint4(p[0], p[1], p[2], p[3]);
-    }
-    act = out;
-    as = FF_HS;
-    kin = MLP_HID;
+    fb_store(h, (l & 1) ? Hs1 : Hs0, A.HT[l], A.ld, m0, wave, r16, q);
+    ww.store((l & 1) ? WA : WB, nnext, MLP_HID);
+    lds_barrier();
   }
-  // output layer: 16 columns (3 used), no ReLU, FP32 y
-  __syncthreads();
-  for (int v = tid; v < MLP_OUTPAD * (MLP_HID / 8); v += 256) {
-    const int r = v / (MLP_HID / 8), kk = (v % (MLP_HID / 8)) * 8;
-    *(uint4*)&Ws[r * FF_HS + kk] = *(const uint4*)&A.w[MLP_HIDDEN_LAYERS][(size_t)r * MLP_HID + kk];
-  }
-  __syncthreads();
-  {
-    f32x4_t acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // ---- output layer: 16 columns (3 used), no ReLU, FP32 y; waves 0..3 take
+  // an m-tile each.  H_4 is in Hs1, W_5 in WA; W_5^T goes to WB, its K of 16
+  // zero-padded to 32
+  ww.load(A.wbt[MLP_HIDDEN_LAYERS], MLP_HID, MLP_OUTPAD);
+  if (wave < 4) {
+    f32x4_t o = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     for (int ks = 0; ks < MLP_HID; ks += 32) {
-      const uint4 va = *(const uint4*)&act[(16 * wave + r16) * FF_HS + ks + 8 * q];
-      const uint4 vb = *(const uint4*)&Ws[r16 * FF_HS + ks + 8 * q];
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&va, *(const bf16x8_t*)&vb, acc, 0, 0, 0);
+      const uint4 va = *(const uint4*)&Hs1[(16 * wave + r16) * FF_HS + ks + 8 * q];
+      const uint4 vb = *(const uint4*)&WA[r16 * FF_HS + ks + 8 * q];
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&va, *(const bf16x8_t*)&vb, o, 0, 0, 0);
     }
     const float bias = A.b[MLP_HIDDEN_LAYERS][r16];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = 16 * wave + 4 * q + e;
-      const float v = acc[e] + bias;
-      ys[m * MLP_OUTPAD + r16] = v;
-      if (m0 + (uint32_t)m < rows) A.y[(size_t)(m0 + m) * MLP_OUTPAD + r16] = v;
+    for (int e = 0; e < 4; ++e)
+      if (r16 < MLP_OUT) ys[(16 * wave + 4 * q + e) * FB_YS + r16] = o[e] + bias;
+  }
+  ww.store(WB, MLP_HID, MLP_OUTPAD);
+  if (tid < MLP_HID * 2) *(uint4*)&WB[(tid >> 1) * FF_HS + MLP_OUTPAD + (tid & 1) * 8] = make_uint4(0u, 0u, 0u, 0u);
+  lds_barrier();
+  // ---- loss gradient and error bins, the last wave's lanes the rows; dy (zero
+  // past the batch and in the padding columns) into Hs0
+  WStage wn;
+  wn.load(A.wbt[MLP_HIDDEN_LAYERS - 1], MLP_HID, MLP_HID);
+  float e2 = 0.0f;
+  if (wave == 15) {
+    const float inv = 2.0f / (float)((int)rows * MLP_OUT);
+    uint16_t g[MLP_OUT] = {0, 0, 0};
+    if (ok) {
+#pragma unroll
+      for (int c = 0; c < MLP_OUT; ++c) {
+        const float d = ys[lane * FB_YS + c] - ts[lane * FB_YS + c];
+        e2 += d * d;
+        g[c] = f32_to_bf16(d * inv);
+      }
+    }
+    *(uint4*)&Hs0[lane * FF_HS] = make_uint4((uint32_t)g[0] | ((uint32_t)g[1] << 16), (uint32_t)g[2], 0u, 0u);
+#pragma unroll
+    for (int j = 8; j < 32; j += 8) *(uint4*)&Hs0[lane * FF_HS + j] = make_uint4(0u, 0u, 0u, 0u);
+    if (ok) {
+#pragma unroll
+      for (int c = 0; c < MLP_OUT; ++c) A.dyT[(size_t)c * A.ld + m0 + (uint32_t)lane] = g[c];
+      A.row_err[m0 + (uint32_t)lane] = e2;
     }
   }
-  __syncthreads();
-  // loss gradient and error bins, one thread per row
-  if (tid < 64 && m0 + (uint32_t)tid < rows) {
-    const uint32_t r = m0 + (uint32_t)tid;
-    float e2 = 0.0f;
-    const float inv = 2.0f / (float)((int)rows * MLP_OUT);
-    for (int c = 0; c < MLP_OUTPAD; ++c) {
-      float gr = 0.0f;
-      if (c < MLP_OUT) {
-        const float t = log_(1.0f + fmax_(A.target[(size_t)r * MLP_OUT + c], 0.0f));
-        const float d = ys[tid * MLP_OUTPAD + c] - t;
-        e2 += d * d;
-        gr = d * inv;
+  lds_barrier();
+  if (wave == 15 && ok && A.esum) {
+    const float e = e2 < 1e6f ? e2 : 1e6f;
+    atomicAdd(&A.esum[cell], (unsigned long long)(e * 16777216.0f));
+    atomicAdd(&A.ecnt[cell], 1u);
+  }
+  // ---- backward: W_l^T alternately in WB (l = 4, 2) and WA (l = 3, 1), the
+  // deltas in Hs0 (D_4 = dy, D_2) and Hs1 (D_3, D_1)
+#pragma unroll
+  for (int l = MLP_HIDDEN_LAYERS; l >= 1; --l) {
+    const bool even = (l & 1) == 0;
+    fb_product(even ? Hs0 : Hs1, FF_HS, even ? WB : WA, FF_HS, l == MLP_HIDDEN_LAYERS ? 32 : MLP_HID, wave, r16, q, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const uint32_t b = mask >> (8 * (l - 1) + 4 * t + e);
+        h[t][e >> 1] = bf16_pair(b & 1u ? acc[t][e] : 0.0f, b & 2u ? acc[t][e + 1] : 0.0f);
       }
-      const uint16_t h = f32_to_bf16(gr);
-      A.dy[(size_t)r * MLP_OUTPAD + c] = h;
-      A.dyT[(size_t)c * A.ld + r] = h;
-    }
-    A.row_err[r] = e2;
-    if (A.esum) {
-      const uint32_t cell = err_cell(A.in + (size_t)r * MLP_IN);
-      const float e = e2 < 1e6f ? e2 : 1e6f;
-      atomicAdd(&A.esum[cell], (unsigned long long)(e * 16777216.0f));
-      atomicAdd(&A.ecnt[cell], 1u);
+    fb_store(h, l > 1 ? (even ? Hs1 : Hs0) : nullptr, A.dT[l - 1], A.ld, m0, wave, r16, q);
+    if (l > 1) {
+      wn.store(even ? WA : WB, MLP_HID, MLP_HID);
+      if (l > 2) wn.load(A.wbt[l - 2], MLP_HID, MLP_HID);
+      lds_barrier();
     }
   }
 }
 
-// ---------------------------------------------------------------- fused deltas
-// The deltas of the four hidden layers of a training batch in one launch: a
-// workgroup takes 64 rows from dy down to layer 0, D_{l-1} = (D_l . W_l) x
-// [H_{l-1} > 0] with D_4 = dy, the deltas in LDS and each written transposed
-// (dT[l - 1], the weight-gradient operand).  Every product is k_gemm_nt's
-// (dy's 16 columns zero-padded to one K step of 32, the mask applied to the
-// FP32 sum before the BF16 rounding), so the outputs equal those of one launch
-// per layer bit for bit.  A wave computes the tile's 64 rows x 32 of the 128
-// columns.
-constexpr size_t FB_LDS = 2u * (2u * 64u * FF_HS + 128u * FF_HS + 64u * FF_HS);
+// ---------------------------------------------------------------- weight gradients
+// The five layers' dW_l [nout x kin] = A [nout x rows] . B [kin x rows]^T in
+// one launch, the rows split into slices: a workgroup of 8 waves takes one
+// slice of a layer's whole output (two halves of kin for layer 0), so an
+// operand is read once per slice, and writes the FP32 partial; the first half
+// also the row sums of A (the bias gradients), summed in ascending k.  K is
+// staged through LDS 128 at a time; the next stage's loads are in registers
+// while the current one is multiplied.  64x64 tiles of 4 waves without the
+// prefetch took 17 us for 8,192 rows and 96 us for 65,536.
+constexpr int WG_THREADS = 512;
+constexpr int WG_KC = 128;
+constexpr int WG_LS = WG_KC + 8;  // LDS row length (bf16), padded
+constexpr int WG_VEC = 2 * 128 * (WG_KC / 8) / WG_THREADS;  // 16-byte vectors per thread and stage
 
-struct BwdArgs {
-  const uint16_t* dy;                    // [rows x OUTPAD]
-  uint32_t rows;
-  const uint16_t* wbt[MLP_LAYERS];       // W_l^T [kin x nout]
-  const uint16_t* H[MLP_HIDDEN_LAYERS];  // [rows x HID], the ReLU masks
-  uint16_t* dT[MLP_HIDDEN_LAYERS];       // [HID x ld]
-  uint32_t ld;
+struct WgradArgs {
+  const uint16_t* A[MLP_LAYERS];  // D_l^T [nout x ld]
+  const uint16_t* B[MLP_LAYERS];  // X^T or H_{l-1}^T [kin x ld]
+  float* part[MLP_LAYERS];        // [slices][nout][kin]
+  float* bpart[MLP_LAYERS];       // [slices][nout]
+  uint32_t rows, ld, kps;         // kps: rows per slice
+  int slices;
 };
 
-__global__ void __launch_bounds__(256) k_bwd_fused(BwdArgs A) {
-  extern __shared__ __align__(16) unsigned char fl[];
-  uint16_t* const D0 = (uint16_t*)fl;         // [64][FF_HS]: the deltas, ping-pong
-  uint16_t* const D1 = D0 + 64 * FF_HS;
-  uint16_t* Ws = D0 + 2 * 64 * FF_HS;         // [128][FF_HS]
-  uint16_t* Ms = Ws + 128 * FF_HS;                                 // [64][FF_HS]
-  const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6, r16 = lane & 15, q = lane >> 4;
-  const uint32_t m0 = blockIdx.x * 64u;
-  const uint32_t rows = A.rows;
-  // dy rows of the tile: 16 columns, then zeros to 32 (zero past the batch)
-  for (int v = tid; v < 64 * 4; v += 256) {
-    const int r = v >> 2, j = (v & 3) * 8;
-    uint4 val = make_uint4(0u, 0u, 0u, 0u);
-    if (j < MLP_OUTPAD && m0 + (uint32_t)r < rows) val = *(const uint4*)&A.dy[(size_t)(m0 + r) * MLP_OUTPAD + j];
-    *(uint4*)&D0[r * FF_HS + j] = val;
+// Stage vector j of this thread: rows [0, M) of A, then N rows of B, k0 .. k0 + 127.
+__device__ __forceinline__ uint4 wg_load(const uint16_t* A, int M, const uint16_t* B, int N, uint32_t ld, int j,
+                                         uint32_t k0, uint32_t k_end) {
+  const int i = (int)threadIdx.x + j * WG_THREADS, r = i / (WG_KC / 8), kk = (i % (WG_KC / 8)) * 8;
+  uint4 q = make_uint4(0u, 0u, 0u, 0u);
+  const uint16_t* row = r < 128 ? (r < M ? A + (size_t)r * ld : nullptr) : (r - 128 < N ? B + (size_t)(r - 128) * ld : nullptr);
+  const uint32_t k = k0 + (uint32_t)kk;
+  if (row && k + 8u <= k_end) {
+    q = *(const uint4*)&row[k];
+  } else if (row && k < k_end) {
+    uint32_t e[8];
+#pragma unroll
+    for (uint32_t t = 0; t < 8; ++t) e[t] = k + t < k_end ? row[k + t] : 0u;
+    q = make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
   }
-  const uint16_t* act = D0;
-  for (int l = MLP_HIDDEN_LAYERS; l >= 1; --l) {
-    const int nout = l == MLP_HIDDEN_LAYERS ? MLP_OUTPAD : MLP_HID;  // K of this product
-    const int kpad = (nout + 31) / 32 * 32;
-    __syncthreads();  // the previous step is done with Ws and Ms
-    // W_l^T [128 x nout], zero-padded to kpad columns
-    for (int v = tid; v < MLP_HID * (kpad / 8); v += 256) {
-      const int r = v / (kpad / 8), j = (v % (kpad / 8)) * 8;
-      uint4 val = make_uint4(0u, 0u, 0u, 0u);
-      if (j < nout) val = *(const uint4*)&A.wbt[l][(size_t)r * nout + j];
-      *(uint4*)&Ws[r * FF_HS + j] = val;
+  return q;
+}
+
+__global__ void __launch_bounds__(WG_THREADS) k_wgrad(WgradArgs g) {
+  __shared__ __align__(16) uint16_t S[256 * WG_LS];  // rows 0..127: A, 128..255: B
+  const int lane = lane_id(), wave = (int)(threadIdx.x >> 6), r16 = lane & 15, q = lane >> 4;
+  // products: layer 0's two halves, then layers 1..4; slices fastest
+  const int z = (int)blockIdx.x % g.slices, prod = (int)blockIdx.x / g.slices;
+  const int l = prod < 2 ? 0 : prod - 1, n0 = prod == 1 ? MLP_KPAD / 2 : 0;
+  const int M = l == MLP_HIDDEN_LAYERS ? MLP_OUTPAD : MLP_HID, kin = l == 0 ? MLP_KPAD : MLP_HID;
+  const int N = l == 0 ? MLP_KPAD / 2 : MLP_HID;
+  const uint16_t* A = g.A[l];
+  const uint16_t* B = g.B[l] + (size_t)n0 * g.ld;
+  const uint32_t k_begin = (uint32_t)z * g.kps, k_end = min(g.rows, k_begin + g.kps);
+  // wave: m-tiles 4 (wave / 4) + 0..3, n-tiles 2 (wave % 4) + 0..1 (with one
+  // m-tile, the output layer: m-tile 0, n-tile wave)
+  const bool thin = M == MLP_OUTPAD;
+  const int mt = thin ? 0 : 4 * (wave >> 2), nt = thin ? wave : 2 * (wave & 3);
+  f32x4_t acc[4][2];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float rowsum = 0.0f;
+  const bool want_rowsum = n0 == 0 && (int)threadIdx.x < M;
+  uint4 v[WG_VEC];
+  if (k_begin < k_end) {
+#pragma unroll
+    for (int j = 0; j < WG_VEC; ++j) v[j] = wg_load(A, M, B, N, g.ld, j, k_begin, k_end);
+  }
+  for (uint32_t k0 = k_begin; k0 < k_end; k0 += WG_KC) {
+    lds_barrier();  // the previous stage has been read
+#pragma unroll
+    for (int j = 0; j < WG_VEC; ++j) {
+      const int i = (int)threadIdx.x + j * WG_THREADS;
+      *(uint4*)&S[(i / (WG_KC / 8)) * WG_LS + (i % (WG_KC / 8)) * 8] = v[j];
     }
-    // the mask rows H_{l-1}
-    for (int v = tid; v < 64 * (MLP_HID / 8); v += 256) {
-      const int r = v / (MLP_HID / 8), j = (v % (MLP_HID / 8)) * 8;
-      uint4 val = make_uint4(0u, 0u, 0u, 0u);
-      if (m0 + (uint32_t)r < rows) val = *(const uint4*)&A.H[l - 1][(size_t)(m0 + r) * MLP_HID + j];
-      *(uint4*)&Ms[r * FF_HS + j] = val;
+    lds_barrier();
+    if (k0 + WG_KC < k_end) {
+#pragma unroll
+      for (int j = 0; j < WG_VEC; ++j) v[j] = wg_load(A, M, B, N, g.ld, j, k0 + WG_KC, k_end);
     }
-    __syncthreads();
-    f32x4_t acc[4][2];
+    const int kc = (int)min((uint32_t)WG_KC, (k_end - k0 + 31u) / 32u * 32u);
+    for (int ks = 0; ks < kc; ks += 32) {
+      uint4 af[4], bf[2];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+      for (int b = 0; b < 2; ++b)
+        if (b == 0 || !thin) bf[b] = *(const uint4*)&S[(128 + 16 * (nt + b) + r16) * WG_LS + ks + 8 * q];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int ks = 0; ks < kpad; ks += 32) {
-      bf16x8_t af[4], bfr[2];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const uint4 v = *(const uint4*)&act[(16 * a + r16) * FF_HS + ks + 8 * q];
-        af[a] = *(const bf16x8_t*)&v;
-      }
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const uint4 v = *(const uint4*)&Ws[(32 * wave + 16 * b + r16) * FF_HS + ks + 8 * q];
-        bfr[b] = *(const bf16x8_t*)&v;
-      }
+      for (int a = 0; a < 4; ++a)
+        if (a == 0 || !thin) af[a] = *(const uint4*)&S[(16 * (mt + a) + r16) * WG_LS + ks + 8 * q];
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+        for (int b = 0; b < 2; ++b)
+          if ((a == 0 && b == 0) || !thin)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&af[a], *(const bf16x8_t*)&bf[b],
+                                                                acc[a][b], 0, 0, 0);
     }
-    // lane holds D_{l-1}[16a + 4q + e][32 wave + 16b + r16] before the mask
-    uint16_t* out = ((MLP_HIDDEN_LAYERS - l) & 1) ? D0 : D1;
+    if (want_rowsum) {
+      for (int k = 0; k < kc; k += 8) {
+        const uint4 p = *(const uint4*)&S[(int)threadIdx.x * WG_LS + k];
+        const uint32_t w[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          rowsum += u2f(w[t] << 16);
+          rowsum += u2f(w[t] & 0xffff0000u);
+        }
+      }
+    }
+  }
+  // lane holds C[16 (mt + a) + 4q + e][16 (nt + b) + r16]
+  float* P = g.part[l] + (size_t)z * M * kin;
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int n = 32 * wave + 16 * b + r16;
+      if (thin && (a > 0 || b > 0)) continue;
+      const int n = 16 * (nt + b) + r16;
+      if (n >= N) continue;
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int m = 16 * a + 4 * q + e;
-          float v = acc[a][b][e];
-          if (!(bf_to_f(Ms[m * FF_HS + n]) > 0.0f)) v = 0.0f;
-          out[m * FF_HS + n] = f32_to_bf16(v);
-        }
+      for (int e = 0; e < 4; ++e) P[(size_t)(16 * (mt + a) + 4 * q + e) * kin + n0 + n] = acc[a][b][e];
     }
-    __syncthreads();
-    for (int v = tid; v < MLP_HID * 8; v += 256) {
-      const int n = v >> 3, j = (v & 7) * 8;
-      uint32_t p[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        p[t] = (uint32_t)out[(j + 2 * t) * FF_HS + n] | ((uint32_t)out[(j + 2 * t + 1) * FF_HS + n] << 16);
-      *(uint4*)&A.dT[l - 1][(size_t)n * A.ld + m0 + j] = make_uint4(p[0], p[1], p[2], p[3]);
-    }
-    act = out;
-  }
+  if (want_rowsum) g.bpart[l][(size_t)z * M + threadIdx.x] = rowsum;
 }
 
 // The gradients of every layer from the split partials: gw[l][i] = sum over
@@ -583,14 +447,11 @@ __global__ void k_grad_sum(GradSum S) {
   int l = 0;
   while (l + 1 < MLP_LAYERS && t >= S.first[l + 1]) ++l;
   const uint32_t i = t - S.first[l];
-  float s = 0.0f;
   if (i < S.nw[l]) {
-    for (int z = 0; z < S.slices; ++z) s += S.part[l][(size_t)z * S.nw[l] + i];
-    S.gw[l][i] = s;
+    S.gw[l][i] = slice_sum(S.part[l] + i, S.nw[l], S.slices);
   } else {
     const uint32_t m = i - S.nw[l];
-    for (int z = 0; z < S.slices; ++z) s += S.bpart[l][(size_t)z * S.nb[l] + m];
-    S.gb[l][m] = s;
+    S.gb[l][m] = slice_sum(S.bpart[l] + m, S.nb[l], S.slices);
   }
 }
 
@@ -607,54 +468,34 @@ int mlp_train_slices(uint32_t rows) { return (int)std::max<uint32_t>(1u, std::mi
 
 uint32_t mlp_train_ld(uint32_t rows) { return (rows + 63u) / 64u * 64u; }
 
-hipError_t mlp_train_grads(const MlpDev& w, const float* in, uint32_t rows, uint16_t* const* H,
-                           float* y, const float* target, MlpTrainBufs& tb, MlpTrainT& tt, bool reduce,
-                           hipStream_t st, unsigned long long* esum, unsigned int* ecnt) {
+hipError_t mlp_train_grads(const MlpDev& w, const float* in, uint32_t rows, const float* target, MlpTrainBufs& tb,
+                           MlpTrainT& tt, bool reduce, hipStream_t st, unsigned long long* esum, unsigned int* ecnt) {
   if (rows == 0) return hipSuccess;
   const uint32_t ld = tt.ld;
   if (ld < mlp_train_ld(rows)) return hipErrorInvalidValue;
   hipError_t e;
-  // encoding, forward (X^T, H_l and H_l^T, y), the loss gradient and the
-  // error bins: one launch
   {
-    FwdArgs f;
+    FwdBwdArgs f;
     memset(&f, 0, sizeof(f));
-    f.XT = tt.XT;
     f.rows = rows;
+    f.ld = ld;
+    f.in = in;
+    f.target = target;
     for (int l = 0; l < MLP_LAYERS; ++l) {
       f.w[l] = w.wb[l];
+      f.wbt[l] = w.wbt[l];
       f.b[l] = w.b[l];
     }
+    f.XT = tt.XT;
     for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) {
-      f.H[l] = H[l];
       f.HT[l] = tt.HT[l];
+      f.dT[l] = tt.dT[l];
     }
-    f.ld = ld;
-    f.y = y;
-    f.target = target;
-    f.dy = tb.dy;
     f.dyT = tt.dyT;
     f.row_err = tb.row_err;
-    f.in = in;
     f.esum = esum;
     f.ecnt = ecnt;
-    hipLaunchKernelGGL(k_fwd_fused, dim3((rows + 63) / 64), dim3(256), FF_LDS, st, f);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  // backward: the four hidden layers' deltas in one launch, then the five
-  // split weight-gradient products in one launch
-  {
-    BwdArgs bw;
-    memset(&bw, 0, sizeof(bw));
-    bw.dy = tb.dy;
-    bw.rows = rows;
-    for (int l = 0; l < MLP_LAYERS; ++l) bw.wbt[l] = w.wbt[l];
-    for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) {
-      bw.H[l] = H[l];
-      bw.dT[l] = tt.dT[l];
-    }
-    bw.ld = ld;
-    hipLaunchKernelGGL(k_bwd_fused, dim3((rows + 63) / 64), dim3(256), FB_LDS, st, bw);
+    hipLaunchKernelGGL(k_fwd_bwd, dim3((rows + 63) / 64), dim3(FB_THREADS), FB_LDS, st, f);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   const int slices = mlp_train_slices(rows);
@@ -662,33 +503,31 @@ hipError_t mlp_train_grads(const MlpDev& w, const float* in, uint32_t rows, uint
   GradSum S;
   memset(&S, 0, sizeof(S));
   S.slices = slices;
-  NtArgs wg[MLP_LAYERS];
-  int wsl[MLP_LAYERS];
+  WgradArgs wg;
+  memset(&wg, 0, sizeof(wg));
+  wg.rows = rows;
+  wg.ld = ld;
+  wg.kps = (uint32_t)kps;
+  wg.slices = slices;
   float* part = tt.part;  // partials of layer 4 first, then 3, ..., 0
   for (int l = MLP_HIDDEN_LAYERS; l >= 0; --l) {
-    const int nout = l == MLP_HIDDEN_LAYERS ? MLP_OUTPAD : MLP_HID;
-    const int kl = l == 0 ? MLP_KPAD : MLP_HID;
-    NtArgs a = nt_args(nout, kl, (int)rows);
-    a.A = l == MLP_HIDDEN_LAYERS ? tt.dyT : tt.dT[l];
-    a.lda = (int)ld;
-    a.B = l == 0 ? tt.XT : tt.HT[l - 1];
-    a.ldb = (int)ld;
-    a.kps = kps;
-    a.part = part;
-    a.bpart = part + (size_t)slices * nout * kl;
-    wg[l] = a;
-    wsl[l] = slices;
-    S.part[l] = a.part;
-    S.bpart[l] = a.bpart;
-    tt.part_w[l] = a.part;
-    tt.part_b[l] = a.bpart;
+    const int nout = mlp_nout(l), kl = mlp_kin(l);
+    wg.A[l] = l == MLP_HIDDEN_LAYERS ? tt.dyT : tt.dT[l];
+    wg.B[l] = l == 0 ? tt.XT : tt.HT[l - 1];
+    wg.part[l] = part;
+    wg.bpart[l] = part + (size_t)slices * nout * kl;
+    S.part[l] = wg.part[l];
+    S.bpart[l] = wg.bpart[l];
+    tt.part_w[l] = wg.part[l];
+    tt.part_b[l] = wg.bpart[l];
     S.gw[l] = tb.gw[l];
     S.gb[l] = tb.gb[l];
     S.nw[l] = (uint32_t)(nout * kl);
     S.nb[l] = (uint32_t)nout;
     part += (size_t)slices * (nout * kl + nout);
   }
-  if ((e = gemm_nt_multi(wg, wsl, st)) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_wgrad, dim3((unsigned)(slices * (MLP_LAYERS + 1))), dim3(WG_THREADS), 0, st, wg);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   tt.slices = slices;
   if (!reduce) return hipSuccess;
   uint32_t tot = 0;
