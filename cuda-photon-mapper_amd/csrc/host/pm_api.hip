@@ -269,6 +269,7 @@ GatherMap gather_map(const pm_context* c, const DevMap& m, int k, float rcap) {
   g.tpayload = m.tpayload;
   g.n = m.n;
   g.nl = m.nl;
+  g.L = m.L;
   g.bf16 = m.bf16;
   g.k = k;
   g.rcap2 = rcap * rcap;
@@ -394,7 +395,7 @@ int pm_destroy(pm_context* c) {
   c->ms.release();
   c->mv.release();
   for (DevBuf* b : {&c->spheres_d, &c->density_d, &c->cnt_s, &c->cnt_v, &c->off_s, &c->off_v, &c->scratch,
-                    &c->scratch2, &c->tally_part, &c->tally9, &c->small, &c->counters, &c->vox_grid_s, &c->vox_grid_v,
+                    &c->scratch2, &c->tally_part, &c->tally9, &c->small, &c->counters, &c->items, &c->vox_grid_s, &c->vox_grid_v,
                     &c->vox_sat_s, &c->vox_sat_v})
     b->release();
   if (c->e0) (void)hipEventDestroy(c->e0);
@@ -428,6 +429,9 @@ int pm_build(pm_context* c) {
   HIPCHK(hipEventRecord(c->ev_join, c->stream2));
   HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
   HIPCHK(hipEventRecord(c->e1, c->stream));
+  // the render's work items: a tile has at least 4 pixels, or the launch is small
+  HIPCHK(c->items.ensure(4ull * packet_item_words((uint32_t)std::max<uint64_t>(
+                             (uint64_t)c->cfg.width * (uint64_t)c->cfg.height / 4u, 1u << 15))));
   HIPCHK(hipStreamSynchronize(c->stream));
   c->stats.ms_build = elapsed_ms(c->e0, c->e1);
   c->built = true;
@@ -478,7 +482,8 @@ int render_crop_impl(pm_context* c, int x0, int y0, int w, int h, float* rgb_dev
   r.gather_mode = c->gather_mode;
   r.tile_regions = c->tile_regions;
   r.sample_lanes = c->sample_lanes;
-  r.top_levels = c->top_levels;
+  r.cus = 256;
+  (void)hipDeviceGetAttribute(&r.cus, hipDeviceAttributeMultiprocessorCount, c->device);
   if (counters) {
     r.counters = counters;
     HIPCHK(launch_fill_u32(reinterpret_cast<uint32_t*>(counters), 0u, 4, c->stream));
@@ -511,22 +516,22 @@ int render_crop_impl(pm_context* c, int x0, int y0, int w, int h, float* rgb_dev
     HIPCHK(launch_render_voxel(r, G, c->stream));
   } else {
   HIPCHK(hipEventRecord(c->e0, c->stream));
-  if (r.gather_mode == 5) {
-    // auto: the two-pass gather (march passes merged, first passes counted)
-    // pays off when the frame keeps many more waves in flight than the 8-byte
-    // heaps allow and the maps are large; small frames or maps run the
-    // one-pass gather
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
-    const uint64_t tiles = (uint64_t)((w + 7) / 8) * (uint64_t)((h + 7) / 8);
-    const uint64_t recs = (uint64_t)c->ms.m.n + (uint64_t)c->mv.m.n;
-    r.gather_mode = tiles >= 16ull * (uint64_t)cus && recs >= (1ull << 20) ? 7 : 1;
-  }
   switch (r.gather_mode) {
     case 0: HIPCHK(launch_render(r, c->stream)); break;
     case 1: HIPCHK(launch_render_lane(r, c->stream)); break;
     case 4: HIPCHK(launch_render_lane4(r, c->stream)); break;
-    case 7: HIPCHK(launch_render_lane7(r, c->stream)); break;
+    // auto: the packet gather, the fastest at every size (one GPU, ms, against
+    // the 8-byte heap: 64x48 room crop 0.4 / 6.1, 256x256 room 3.1 / 14, 477x271x4
+    // fog crop 34 / 467)
+    case 5:
+    case 7:
+      // the work items' scratch: grown here, or as pm_build left it for the
+      // caller that allocates nothing (a larger frame then renders in raster order)
+      if (!counters) HIPCHK(c->items.ensure(4ull * packet_item_words(packet_tiles(r))));
+      r.items.head = c->items.as<uint32_t>();
+      r.items.words = c->items.bytes / 4;
+      HIPCHK(launch_render_packet(r, c->stream));
+      break;
     default: HIPCHK(launch_render_lane2(r, c->stream)); break;
   }
   }
@@ -642,9 +647,7 @@ int pm_set_option(pm_context* c, int option, int value) {
       c->cache.near_groups = value;
       return PM_OK;
     case PM_OPT_TOP_LEVELS:
-      if (value < 0 || value > kMaxTopLevels) return PM_ERR_INVALID;
-      c->top_levels = value;
-      return PM_OK;
+      return value < 0 || value > kMaxTopLevels ? PM_ERR_INVALID : PM_OK;  // no effect: no gather stages tree nodes
     case PM_OPT_VOXEL_GRID:
       if (value < 0 || value > 2) return PM_ERR_INVALID;
       c->voxel_grid = value;

@@ -57,8 +57,14 @@ struct pm_batch {
   std::vector<BatchRenderScene> rsc;
   std::vector<uint64_t> img_off;
   uint64_t npix = 0;
-  std::vector<uint2> items_h;
-  DevBuf rsc_d, items_d, items_tune_d, head, rgb, counters;
+  // work items (scene, tile): of the heap gathers' 8x8 tiles, and of the packet
+  // gather's tiles, whose shape depends on the scene
+  struct WorkList {
+    std::vector<uint2> h;
+    DevBuf d, tune_d;  // every item; the autotuner's subset
+  } work[2];
+  WorkList& items() { return work[tune.gather_mode == 7 ? 1 : 0]; }
+  DevBuf rsc_d, head, rgb, counters;
   int fp64 = 0, cone = 0, kmax = 1, cus = 1, grid = 1;
   pm_batch_tuning tune;
   // graph
@@ -205,6 +211,7 @@ GatherMap tree_gather_map(const pm_batch* b, int scene, int vol, uint32_t tree) 
   g.tpayload = b->tpayload.p ? (const char*)b->tpayload.p + stride * b->tree_pbase_h[tree] : nullptr;
   g.n = b->tree_n[tree];
   g.nl = b->tree_nl[tree];
+  g.L = (uint32_t)b->L;
   g.bf16 = b->bf16;
   g.k = vol ? c.k_volume : c.k_surface;
   const float rc = vol ? c.rcap_volume : c.rcap_surface;
@@ -214,6 +221,18 @@ GatherMap tree_gather_map(const pm_batch* b, int scene, int vol, uint32_t tree) 
 }
 
 int setup_scene_maps(pm_batch* b);
+
+// log2 of the packet gather's march lanes in scene s.
+int batch_march_lanes(const pm_batch* b, int s) {
+  uint64_t pixels = 0;
+  for (const pm_config& c : b->cfg) pixels += (uint64_t)c.width * (uint64_t)c.height;
+  GatherMap gv;
+  memset(&gv, 0, sizeof(gv));
+  gv.n = b->nrec_v[s];
+  gv.k = b->cfg[s].k_volume;
+  gv.rcap2 = b->cfg[s].rcap_volume * b->cfg[s].rcap_volume;
+  return packet_march_lanes_batch(render_params(b->cfg[s]), gv, pixels, b->cus);
+}
 
 // Forest tables for leaf size L, the per-scene gather maps, the build scratch.
 int setup_forest(pm_batch* b, int L) {
@@ -349,6 +368,7 @@ int setup_scene_maps(pm_batch* b) {
     r.exposure = c.exposure;
     r.w = c.width;
     r.h = c.height;
+    r.lu = batch_march_lanes(b, s);
     r.img_off = b->img_off[s];
   }
   HIPCHK(b->rsc_d.ensure(sizeof(BatchRenderScene) * b->ns));
@@ -356,7 +376,7 @@ int setup_scene_maps(pm_batch* b) {
   return PM_OK;
 }
 
-// Image arena and the work list: the 8x8 tiles of every scene, scenes in
+// Image arena and the work lists: the tiles of every scene, scenes in
 // decreasing order of expected cost per tile (march length x log of the map
 // sizes x k), so the persistent grid ends on the cheapest tiles.
 int setup_render(pm_batch* b) {
@@ -374,14 +394,49 @@ int setup_render(pm_batch* b) {
     order[s] = s;
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return cost[a] > cost[c]; });
-  b->items_h.clear();
+  b->work[0].h.clear();
+  b->work[1].h.clear();
+  std::vector<uint2> light;
+  DevBuf items;
+  struct Release {
+    DevBuf& d;
+    ~Release() { d.release(); }
+  } release{items};
   for (int s : order) {
     const pm_config& c = b->cfg[s];
     const uint32_t tiles = ceil_div(c.width, 8) * ceil_div(c.height, 8);
-    for (uint32_t t = 0; t < tiles; ++t) b->items_h.push_back(make_uint2((uint32_t)s, t));
+    for (uint32_t t = 0; t < tiles; ++t) b->work[0].h.push_back(make_uint2((uint32_t)s, t));
+    // the packet gather's items: every scene's heavy tiles (k_packet_tiles)
+    // before all light ones (16 scenes 30.0 -> 27.5 ms).  Not split: the launch
+    // has many of them, and quarters of more march lanes cost more than the
+    // tail (45 ms)
+    RenderLaunch r;
+    memset(&r, 0, sizeof(r));
+    r.sc = b->tsc[s].sc;
+    r.rp = render_params(c);
+    r.w = c.width;
+    r.h = c.height;
+    r.cus = b->cus;
+    const int lu = batch_march_lanes(b, s), lp = 6 - lu;
+    const uint32_t n = ceil_div(c.width, pk_tile_w(lp)) * ceil_div(c.height, pk_tile_h(lp));
+    HIPCHK(items.ensure(4ull * packet_item_words(n)));
+    r.items.head = items.as<uint32_t>();
+    HIPCHK(launch_packet_tiles(r, lu, 0, n, b->stream));
+    std::vector<uint32_t> h(packet_item_words(n));
+    HIPCHK(hipMemcpyAsync(h.data(), r.items.head, 4ull * h.size(), hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    std::sort(h.begin() + 4, h.begin() + 4 + h[1]);
+    std::sort(h.begin() + 4 + 4ull * n, h.begin() + 4 + 4ull * n + h[2]);
+    for (uint32_t i = 0; i < h[1]; i += lp >= 2 ? 4 : 1)
+      b->work[1].h.push_back(make_uint2((uint32_t)s, h[4 + i] >> 2));
+    for (uint32_t i = 0; i < h[2]; ++i)
+      light.push_back(make_uint2((uint32_t)s, h[4 + 4ull * n + i]));
   }
-  HIPCHK(b->items_d.ensure(sizeof(uint2) * std::max<size_t>(b->items_h.size(), 1)));
-  HIPCHK(hipMemcpy(b->items_d.p, b->items_h.data(), sizeof(uint2) * b->items_h.size(), hipMemcpyHostToDevice));
+  b->work[1].h.insert(b->work[1].h.end(), light.begin(), light.end());
+  for (pm_batch::WorkList& W : b->work) {
+    HIPCHK(W.d.ensure(sizeof(uint2) * std::max<size_t>(W.h.size(), 1)));
+    HIPCHK(hipMemcpy(W.d.p, W.h.data(), sizeof(uint2) * W.h.size(), hipMemcpyHostToDevice));
+  }
   HIPCHK(b->rgb.ensure(12 * std::max<uint64_t>(b->npix, 1)));
   HIPCHK(b->head.ensure(16));
   HIPCHK(b->counters.ensure(16));
@@ -390,7 +445,7 @@ int setup_render(pm_batch* b) {
 
 int set_grid(pm_batch* b) {
   const int occ = render_batch_occupancy(b->fp64, b->cone, b->tune.block_threads, b->tune.heap_slots,
-                                         b->tune.heap_key_bytes, b->tune.gather_mode == 7, b->tune.top_levels);
+                                         b->tune.heap_key_bytes, b->tune.gather_mode == 7);
   if (occ < 1) return PM_ERR_INVALID;
   b->grid = b->cus * occ;
   return PM_OK;
@@ -434,7 +489,6 @@ hipError_t enqueue_frame(pm_batch* b, const uint2* items, uint32_t nitems, hipEv
   R.heap_slots = b->tune.heap_slots;
   R.key_bytes = b->tune.heap_key_bytes;
   R.counting = b->tune.gather_mode == 7;
-  R.top_levels = b->tune.top_levels;
   hipError_t e;
   if ((e = launch_trace_count_batch(b->tsc_d.as<BatchTraceScene>(), b->block_scene_d.as<uint32_t>(), b->tblocks,
                                     b->cnt_s.as<uint32_t>(), b->cnt_v.as<uint32_t>(), st)) != hipSuccess)
@@ -485,7 +539,7 @@ hipError_t enqueue_frame(pm_batch* b, const uint2* items, uint32_t nitems, hipEv
 int capture(pm_batch* b) {
   release_graph(b);
   HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-  hipError_t e = enqueue_frame(b, b->items_d.as<uint2>(), (uint32_t)b->items_h.size(), nullptr, nullptr);
+  hipError_t e = enqueue_frame(b, b->items().d.as<uint2>(), (uint32_t)b->items().h.size(), nullptr, nullptr);
   hipGraph_t g = nullptr;
   hipError_t e2 = hipStreamEndCapture(b->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -561,7 +615,8 @@ void destroy(pm_batch* b) {
                     &b->off_v, &b->scan_tmp, &b->small, &b->tally_part, &b->tally9, &b->x, &b->y, &b->z,
                     &b->payload, &b->tpts, &b->nodes, &b->nrange, &b->point_tree, &b->tree_pbase, &b->tree_root,
                     &b->node_lo, &b->node_hi, &b->node_lc, &b->node_lb, &b->node_child, &b->node_pbase,
-                    &b->level_nodes, &b->build_tmp, &b->rsc_d, &b->items_d, &b->items_tune_d, &b->head, &b->rgb,
+                    &b->level_nodes, &b->build_tmp, &b->rsc_d, &b->work[0].d, &b->work[0].tune_d,
+                    &b->work[1].d, &b->work[1].tune_d, &b->head, &b->rgb,
                     &b->counters, &b->bmin, &b->bmax, &b->tpayload, &b->tree_desc_d, &b->leaf_pref_d,
                     &b->level_pref_d})
     d->release();
@@ -637,9 +692,9 @@ int pm_batch_create(const pm_config* cfgs, int n, pm_batch** out) {
   pm_batch_tuning t;
   t.leaf_size = 32;
   t.block_threads = 64;
-  t.heap_slots = b->kmax <= 32 ? 32 : 64;
+  t.heap_slots = 64;
   t.heap_key_bytes = 2;
-  t.gather_mode = 0;
+  t.gather_mode = 7;
   t.top_levels = 0;
   int r = setup_scenes(b);
   if (r == PM_OK) r = size_records(b);
@@ -651,7 +706,7 @@ int pm_batch_create(const pm_config* cfgs, int n, pm_batch** out) {
   }
   b->st.ms_setup = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   b->st.n_scenes = (uint32_t)n;
-  b->st.work_items = (uint32_t)b->items_h.size();
+  b->st.work_items = (uint32_t)b->work[0].h.size();
   for (int i = 0; i < n; ++i) b->st.photons += cfgs[i].n_emit;
   b->st.surface_records = b->S_tot;
   b->st.volume_records = b->V_tot;
@@ -674,11 +729,16 @@ int pm_batch_set_tuning(pm_batch* b, const pm_batch_tuning* t) {
 
 int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out, double* best_ms_out) {
   if (!b || sample_stride < 1) return PM_ERR_INVALID;
-  std::vector<uint2> sub;
-  for (size_t i = 0; i < b->items_h.size(); i += (size_t)sample_stride) sub.push_back(b->items_h[i]);
-  HIPCHK(b->items_tune_d.ensure(sizeof(uint2) * std::max<size_t>(sub.size(), 1)));
-  if (!sub.empty())
-    HIPCHK(hipMemcpy(b->items_tune_d.p, sub.data(), sizeof(uint2) * sub.size(), hipMemcpyHostToDevice));
+  uint32_t nsub[2];
+  for (int packet = 0; packet < 2; ++packet) {
+    pm_batch::WorkList& W = b->work[packet];
+    std::vector<uint2> sub;
+    for (size_t i = 0; i < W.h.size(); i += (size_t)sample_stride) sub.push_back(W.h[i]);
+    HIPCHK(W.tune_d.ensure(sizeof(uint2) * std::max<size_t>(sub.size(), 1)));
+    if (!sub.empty())
+      HIPCHK(hipMemcpy(W.tune_d.p, sub.data(), sizeof(uint2) * sub.size(), hipMemcpyHostToDevice));
+    nsub[packet] = (uint32_t)sub.size();
+  }
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   struct EvGuard {
     hipEvent_t* e;
@@ -691,7 +751,7 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
   // objective: kd-build + sampled render (the emission does not depend on the tuning)
   auto trial = [&](double* ms) -> int {
     HIPCHK(hipEventRecord(ev[0], b->stream));
-    HIPCHK(enqueue_frame(b, b->items_tune_d.as<uint2>(), (uint32_t)sub.size(), ev[1], ev[2]));
+    HIPCHK(enqueue_frame(b, b->items().tune_d.as<uint2>(), nsub[b->tune.gather_mode == 7 ? 1 : 0], ev[1], ev[2]));
     HIPCHK(hipEventRecord(ev[3], b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
     float t = 0.0f;
@@ -718,7 +778,6 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
     return PM_OK;
   };
   const int keyb[3] = {8, 4, 2}, slots[2] = {32, 64}, leaves[4] = {4, 8, 16, 32}, blocks[3] = {64, 128, 256};
-  const int tops[4] = {0, 3, 5, 7};
   const pm_batch_tuning start = b->tune;
   for (int kb : keyb)
     for (int sl : slots) {
@@ -730,7 +789,7 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
       int r = consider(t);
       if (r != PM_OK) return r;
     }
-  {  // gather mode 7 (2-byte keys, 64 slots of LDS for its counters)
+  {  // the packet gather
     pm_batch_tuning t = start;
     t.heap_key_bytes = 2;
     t.heap_slots = 64;
@@ -755,16 +814,6 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
     int r = consider(t);
     if (r != PM_OK) return r;
   }
-  if (best.gather_mode == 7) {  // LDS tile: top-of-tree levels staged per wave (mode 7 reads them)
-    const pm_batch_tuning s3 = best;
-    for (int lv : tops) {
-      if (lv == s3.top_levels) continue;
-      pm_batch_tuning t = s3;
-      t.top_levels = lv;
-      int r = consider(t);
-      if (r != PM_OK) return r;
-    }
-  }
   int r = apply_tuning(b, best, true);
   if (r != PM_OK) return r;
   if (best_out) *best_out = best;
@@ -786,7 +835,7 @@ int pm_batch_submit(pm_batch* b) {
   HIPCHK(hipMemcpy(b->tally.data(), b->tally9.p, sizeof(double) * 9 * b->ns, hipMemcpyDeviceToHost));
   pm_batch_stats& s = b->st;
   s.n_scenes = (uint32_t)b->ns;
-  s.work_items = (uint32_t)b->items_h.size();
+  s.work_items = (uint32_t)b->work[0].h.size();
   s.photons = 0;
   for (int i = 0; i < b->ns; ++i) s.photons += b->cfg[i].n_emit;
   s.surface_records = b->S_tot;
@@ -812,7 +861,7 @@ int pm_batch_time_phases(pm_batch* b, double* ms_emit, double* ms_build, double*
   for (int i = 0; i < 4; ++i) HIPCHK(hipEventCreate(&ev[i]));
   // the graph's kernels, launched one by one on the batch stream
   HIPCHK(hipEventRecord(ev[0], b->stream));
-  HIPCHK(enqueue_frame(b, b->items_d.as<uint2>(), (uint32_t)b->items_h.size(), ev[1], ev[2]));
+  HIPCHK(enqueue_frame(b, b->items().d.as<uint2>(), (uint32_t)b->items().h.size(), ev[1], ev[2]));
   HIPCHK(hipEventRecord(ev[3], b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
   float t[3] = {0.0f, 0.0f, 0.0f};

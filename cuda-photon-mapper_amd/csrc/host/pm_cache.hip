@@ -132,7 +132,7 @@ void cache_release(CacheState& k) {
   for (DevBuf* b : {&k.params, &k.grads, &k.adam_m, &k.adam_v, &k.params_bf16, &k.params_ema, &k.ema_bf16, &k.X, &k.y, &k.H[0], &k.H[1],
                     &k.row_err, &k.rgb, &k.err_sum, &k.err_cnt, &k.rec_cnt, &k.rec_off, &k.rec_in,
                     &k.rec_wt, &k.rec_code, &k.rec_val, &k.sel_in, &k.sel_t, &k.list, &k.list_cnt, &k.cell_fb,
-                    &k.row_code, &k.row_list, &k.loss_part, &k.loss_acc, &k.rec_q, &k.map_hash, &k.list_fb,
+                    &k.row_code, &k.row_list, &k.loss_part, &k.loss_acc, &k.rec_q, &k.map_hash, &k.list_fb, &k.sel_order,
                     &k.XT, &k.dT[0], &k.dT[1], &k.dT[2], &k.dT[3], &k.dyT, &k.tpart})
     b->release();
   for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) k.HT[l].release();
@@ -413,8 +413,18 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   HIPCHK(c->small.ensure(64));
   unsigned long long* ntot_dev = (unsigned long long*)(c->small.as<uint32_t>() + 14);
   HIPCHK(launch_count_total(k.rec_cnt.as<uint32_t>(), npix, ntot_dev, st));
+  // exact values with the gather of mode 7 under modes 7 and 5 (auto)
+  const int mode7 = c->gather_mode == 7 || c->gather_mode == 5 ? 1 : 0;
   uint64_t N = 0;
+  unsigned long long hh[2] = {0ull, 0ull};  // the maps' fingerprints (prepare_seeds), in the same read-back
   HIPCHK(hipMemcpyAsync(&N, ntot_dev, 8, hipMemcpyDeviceToHost, st));
+  if (mode7 && k.use_seeds) {
+    HIPCHK(k.map_hash.ensure(16));
+    unsigned long long* mh = (unsigned long long*)k.map_hash.p;
+    HIPCHK(launch_point_hash(c->ms.m.tpts, c->ms.m.n, mh, st));
+    HIPCHK(launch_point_hash(c->mv.m.tpts, c->mv.m.n, mh + 1, st));
+    HIPCHK(hipMemcpyAsync(hh, mh, 16, hipMemcpyDeviceToHost, st));
+  }
   HIPCHK(hipStreamSynchronize(st));
   if (N >= 0xffffffffull) return PM_ERR_CAPACITY;
   HIPCHK(k.rec_in.ensure(4ull * MLP_IN * std::max<uint64_t>(N, 1)));
@@ -431,8 +441,6 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   // 4: online training on a subset with exact kNN targets
   GatherMap gs = make_gather_map(c, c->ms.m, c->cfg.k_surface, c->cfg.rcap_surface);
   GatherMap gv = make_gather_map(c, c->mv.m, c->cfg.k_volume, c->cfg.rcap_volume);
-  // exact values with the gather of mode 7 under modes 7 and 5 (auto)
-  const int mode7 = c->gather_mode == 7 || c->gather_mode == 5 ? 1 : 0;
   const uint32_t ncell = 2u * CACHE_GRID * CACHE_GRID * CACHE_GRID;
   HIPCHK(k.err_sum.ensure(8ull * ncell));
   HIPCHK(k.err_cnt.ensure(4ull * ncell));
@@ -456,13 +464,6 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   auto prepare_seeds = [&]() -> int {
     if (seeds_checked || !mode7 || !k.use_seeds) return PM_OK;
     seeds_checked = true;
-    HIPCHK(k.map_hash.ensure(16));
-    unsigned long long* mh = (unsigned long long*)k.map_hash.p;
-    HIPCHK(launch_point_hash(c->ms.m.tpts, c->ms.m.n, mh, st));
-    HIPCHK(launch_point_hash(c->mv.m.tpts, c->mv.m.n, mh + 1, st));
-    unsigned long long hh[2] = {0ull, 0ull};
-    HIPCHK(hipMemcpyAsync(hh, mh, 16, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
     if (k.rec_q_n != N || !k.rec_q.p || hh[0] != k.rec_q_hash[0] || hh[1] != k.rec_q_hash[1]) {
       HIPCHK(k.rec_q.ensure(2ull * std::max<uint64_t>(N, 1)));
       HIPCHK(hipMemsetAsync(k.rec_q.p, 0xff, 2ull * N, st));
@@ -526,6 +527,13 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
       vl.n = S;
       vl.out = k.sel_t.as<float>();
       vl.mode7 = mode7;
+      if (mode7) {  // rows near each other side by side
+        HIPCHK(k.sel_order.ensure(4ull * S));
+        HIPCHK(c->scratch.ensure(4ull * sort_rows_words(S)));
+        HIPCHK(launch_sort_rows(vl.in, S, k.sel_order.as<uint32_t>(), c->scratch.as<uint32_t>(), st));
+        vl.list = k.sel_order.as<uint32_t>();
+        vl.out_by_list = 1;
+      }
       HIPCHK(launch_cache_values(vl, st));
       int r = cache_train_dev(c, k.sel_in.as<float>(), k.sel_t.as<float>(), S, k.batch, k.lr, nullptr,
                               k.err_sum.as<unsigned long long>(), k.err_cnt.as<unsigned int>(), &loss_terms);
@@ -570,6 +578,8 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
     vl.mode7 = mode7;
     vl.kind = kind;
     vl.seed_q = seeds;
+    if (mode7 && kind == 2)
+      HIPCHK(launch_order_rows(vl.in, k.list_fb.as<uint32_t>() + nk2[0], nk2[1], st));
     HIPCHK(launch_cache_values(vl, st));
   }
   if (surface_early) HIPCHK(hipStreamWaitEvent(st, c->ev_join, 0));

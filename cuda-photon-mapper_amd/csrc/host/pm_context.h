@@ -88,7 +88,8 @@ struct CacheState {
   float ema_decay = 0.95f;  // inference on the moving average of the weights (decay per Adam step), 0: off
   bool ema_stale = true;    // the average must restart at the current weights before its next use
   DevBuf rec_cnt, rec_off, rec_in, rec_wt, rec_code, rec_val, sel_in, sel_t, list, list_cnt, cell_fb;
-  DevBuf list_fb;  // the fallback lists (list keeps the kind lists, which the early surface gather reads)
+  DevBuf list_fb;    // the fallback lists (list keeps the kind lists, which the early surface gather reads)
+  DevBuf sel_order;  // the training rows by position
   pm_cache_stats st;
 };
 
@@ -133,8 +134,8 @@ struct pm_context {
   int tile_regions = 0;  // per-XCD tile regions of the lane render (0: raster order)
   int sample_lanes = 1;  // mode 7: a pixel's samples in adjacent lanes
   int render_media = 1;  // 0: the plain render gathers at surface hits only
-  int top_levels = 0;    // mode 7: kd-tree levels staged in LDS per wave
   int voxel_grid = 0;    // 1: the plain render uses the voxel-grid estimate, 2: with the bilinear blend
+  pm::DevBuf items;       // packet renders' work items
   bool vox_ready = false;  // voxel grids and tables hold the current records
   pm::DevBuf vox_grid_s, vox_grid_v, vox_sat_s, vox_sat_v;
   pm_stats stats;

@@ -9,7 +9,7 @@
 //                       the surface albedo folded in) and record codes (error
 //                       cell, kind, near-light bit: record_code)
 //   4. training       : a Philox-chosen subset of the records gets exact kNN
-//                       targets (k_values7 under gather modes 7 and auto,
+//                       targets (k_values_packet under gather modes 7 and auto,
 //                       k_values otherwise) and trains the MLP (pm_mlp.hip);
 //                       each batch's pre-update errors are binned into a
 //                       16^3 x {surface, volume} grid (by the fused forward
@@ -20,12 +20,12 @@
 //                       the threshold (or that saw no training sample) are
 //                       re-gathered exactly with kNN (k_cell_fb, the lists of
 //                       record_class by k_list_count / k_list_scatter, then
-//                       k_values7 / k_values over the surface rows and the
-//                       volume rows)
+//                       k_values_packet / k_values over the surface rows and
+//                       the volume rows)
 //   7. k_accumulate   : per pixel, compensated sum of weight x value / spp.
 // No reference counterpart (the reference has no cache); the plain path it
 // replaces is photon_mapping_kernel, photonMappingKernel.cu:1409-1462.
-#include "pm_lane_knn5.h"
+#include "pm_lane_knn3.h"
 #include "pm_mlp.h"
 
 namespace pm {
@@ -75,12 +75,13 @@ struct RecordGather {
   float near2;       // squared near-light radius: no merging closer than this to the light
   __device__ void store(uint32_t k, V3f x, V3f d, V3f nrm, V3f w) {
     if (!write) return;
-    size_t i = (size_t)base + k;
-    float* p = in + i * MLP_IN;
-    p[0] = x.x; p[1] = x.y; p[2] = x.z;
-    p[3] = d.x; p[4] = d.y; p[5] = d.z;
-    p[6] = nrm.x; p[7] = nrm.y; p[8] = nrm.z;
-    wt[3 * i] = w.x; wt[3 * i + 1] = w.y; wt[3 * i + 2] = w.z;
+    const size_t i = (size_t)base + k;
+    // whole rows (4-byte aligned) in 16- and 12-byte stores: every store of a
+    // wave goes to 64 lines, so their number is what the record pass pays for
+    const float row[MLP_IN] = {x.x, x.y, x.z, d.x, d.y, d.z, nrm.x, nrm.y, nrm.z};
+    const float w3[3] = {w.x, w.y, w.z};
+    __builtin_memcpy(in + i * MLP_IN, row, sizeof(row));
+    __builtin_memcpy(wt + 3 * i, w3, sizeof(w3));
     code[i] = record_code(x, nrm, light, near2);
   }
   // Writes the open volume record: at the weighted centroid of its points
@@ -172,7 +173,9 @@ __global__ void __launch_bounds__(64) k_rec(CacheRecordLaunch r) {
   if (!r.write) r.counts[pidx] = g.n;
 }
 
-// Exact kNN value (albedo-free for surfaces) of records list[i] (or i).
+// Exact kNN value (albedo-free for surfaces) of records list[i] (or i), with
+// the terms P (pm_estimate.h).
+template <class P>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) k_values(CacheValueLaunch v) {
   extern __shared__ uint32_t heap_lds[];
   const int lane = lane_id();
@@ -180,7 +183,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) k_
   if (i >= v.n) return;
   const uint32_t rec = v.list ? v.list[i] : i;
   const float* p = v.in + (size_t)rec * MLP_IN;
-  LaneGather3<false, 4> g;  // 2-byte heap: 8 KB of LDS per wave
+  LaneGather3<false, 4, P> g;  // 2-byte heap: 8 KB of LDS per wave
   g.gs = v.gs;
   g.gv = v.gv;
   g.hp.H = (uint16_t*)heap_lds;
@@ -197,56 +200,6 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) k_
   v.out[3 * o] = val.x;
   v.out[3 * o + 1] = val.y;
   v.out[3 * o + 2] = val.z;
-}
-
-__device__ __forceinline__ void put_value(const CacheValueLaunch& v, uint32_t o, V3f val) {
-  v.out[3 * (size_t)o] = val.x;
-  v.out[3 * (size_t)o + 1] = val.y;
-  v.out[3 * (size_t)o + 2] = val.z;
-}
-
-// The same values with the gather of mode 7 (pm_lane_knn5.h), one row per
-// lane: a heap pass for Q on the speculative traversal with node boxes, then
-// the second pass (also speculative, from the tree-ordered payload), for
-// surface and volume rows alike.  A row has no previous march point to seed a
-// count window from.  Values equal k_values'.  KIND 1 or 2: every row is a
-// surface or a volume query (the other branch is not compiled in).
-template <int KIND>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) k_values7(CacheValueLaunch v) {
-  extern __shared__ uint32_t heap_lds[];
-  const int lane = lane_id();
-  const uint32_t i = blockIdx.x * 64u + (uint32_t)lane;
-  if (i >= v.n) return;
-  const uint32_t rec = v.list ? v.list[i] : i;
-  const uint32_t o = v.out_by_list ? rec : i;
-  const float* p = v.in + (size_t)rec * MLP_IN;
-  LaneGather5<false, true> g;
-  g.gs = v.gs;
-  g.gv = v.gv;
-  g.hp.H = (uint16_t*)heap_lds;
-  g.hp.lane = lane;
-  g.hp.k = 0;
-  g.hp.size = 0;
-  g.hg_g = v.hg_g;
-  g.nsurf = g.nvol = 0u;
-  g.prev_r = -1.0f;
-  g.pend = false;
-  g.pend_full = false;
-  const V3f one = v3(1.0f, 1.0f, 1.0f);
-  V3f x = v3(p[0], p[1], p[2]), d = v3(p[3], p[4], p[5]), nrm = v3(p[6], p[7], p[8]);
-  V3f c;
-  const bool surf = KIND == 0 ? !(nrm.x == 0.0f && nrm.y == 0.0f && nrm.z == 0.0f) : KIND == 1;
-  // the seed bucket of this record from the previous frame (none: heap pass)
-  using G = LaneGather5<false, true>;
-  const uint32_t seed = v.seed_q ? (uint32_t)v.seed_q[rec] : G::kNoSeed;
-  uint32_t q = G::kNoSeed;
-  if (surf) {
-    c = g.surface_lone(x, nrm, one, seed, &q);
-  } else {
-    c = g.volume_lone(x, d, one, seed, &q);
-  }
-  if (v.seed_q) v.seed_q[rec] = (uint16_t)q;
-  put_value(v, o, c);
 }
 
 // Training subset, stratified by query kind: rows j < count/2 are drawn from
@@ -474,10 +427,9 @@ hipError_t launch_cache_values(const CacheValueLaunch& v, hipStream_t st) {
   if (v.n == 0) return hipSuccess;
   const size_t lds = 64 * 64 * sizeof(uint16_t);  // 2-byte heap of 64 keys per lane
   const dim3 grid((v.n + 63) / 64);
-  if (!v.mode7) hipLaunchKernelGGL(k_values, grid, dim3(64), lds, st, v);
-  else if (v.kind == 1) hipLaunchKernelGGL(k_values7<1>, grid, dim3(64), lds, st, v);
-  else if (v.kind == 2) hipLaunchKernelGGL(k_values7<2>, grid, dim3(64), lds, st, v);
-  else hipLaunchKernelGGL(k_values7<0>, grid, dim3(64), lds, st, v);
+  if (v.mode7) return launch_cache_values_packet(v, st);
+  if (v.kind != 0) hipLaunchKernelGGL(k_values<SumFp64>, grid, dim3(64), lds, st, v);
+  else hipLaunchKernelGGL(k_values<SumTarget>, grid, dim3(64), lds, st, v);
   return hipGetLastError();
 }
 

@@ -53,22 +53,13 @@ struct GatherMap {
   const void* payload;
   const void* tpayload;  // payload in tree order, or null
   uint32_t n, nl;
+  uint32_t L;  // leaf size: every leaf but the last holds L points, in-order
   int bf16;
   int k;
   float rcap2;
   float scale[3];  // light power / n_emit
-  // top-of-tree tile: the first top_count internal nodes' records, staged in
-  // LDS by the gather kernels that take one (0: none, every read from HBM)
-  const KdNode* top_nodes = nullptr;
-  const uint2* top_nrange = nullptr;
-  const float4* top_bmin = nullptr;
-  const float4* top_bmax = nullptr;
-  uint32_t top_count = 0;
 };
-// LDS bytes of a top-of-tree tile of `levels` levels (2^levels - 1 nodes):
-// boxes (2 x 16 B), node record (8 B) and point range (8 B) per node.
-PM_HD size_t top_tile_bytes(int levels) { return levels > 0 ? 48u * (((size_t)1 << levels) - 1u) : 0u; }
-constexpr int kMaxTopLevels = 7;
+constexpr int kMaxTopLevels = 7;  // largest accepted top-of-tree setting (it has no effect)
 
 // scan / sort (pm_scan_sort.hip)
 size_t scan_temp_words(size_t n);
@@ -163,6 +154,15 @@ hipError_t kd_forest_payload(const float4* tpts, const uint32_t* point_tree, con
 // gather (pm_gather.hip)
 hipError_t launch_knn(GatherMap g, const float* q, uint32_t nq, uint32_t* idx, float* d2, uint32_t* count,
                       hipStream_t st);
+// Work items of a packet render, built on the device before it: head[0] is the
+// next item, head[1] and head[2] the heavy and light items there are.
+struct RenderItems {
+  uint32_t* head;   // null: one wave per tile in raster order
+  size_t words;     // words allocated at head
+  uint32_t* heavy;  // 4 x tile + quarter
+  uint32_t* light;  // tile
+};
+size_t packet_item_words(uint32_t tiles);
 struct RenderLaunch {
   Scene sc;
   RenderParams rp;
@@ -174,16 +174,21 @@ struct RenderLaunch {
   uchar4* u8;      // w*h or null
   unsigned long long* counters;  // [surface queries, volume queries]
   int blocks_per_cu;             // persistent grid: workgroups per compute unit
-  int gather_mode;               // 0: wave per query; lane per query: 1 8-byte, 2 4-byte, 3 2-byte heap
+  int gather_mode;               // 0: wave per query; lane per query: 1 8-byte, 2 4-byte, 4 2-byte heap; 7: packet
   int tile_regions;              // lane modes: 0 raster tile order; rx = 1, 2, 4, 8: rx x (8 / rx) per-XCD regions
   int sample_lanes;              // mode 7: a pixel's spp samples in adjacent lanes (spp 2, 4, 8 or 16)
-  int top_levels;                // mode 7: levels of each tree staged in LDS per wave (0: none)
+  int cus;                       // compute units of the device
+  RenderItems items;             // packet gather: scratch for its work items (head, words), or null
 };
 hipError_t launch_render(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_lane(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_lane2(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_lane4(const RenderLaunch& r, hipStream_t st);
-hipError_t launch_render_lane7(const RenderLaunch& r, hipStream_t st);
+hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st);
+// Tiles of a packet render of r, and the lists of its heavy and light items
+// into r.items (head set, packet_item_words(tiles) words).
+uint32_t packet_tiles(const RenderLaunch& r);
+hipError_t launch_packet_tiles(RenderLaunch& r, int lu, int ls, uint32_t tiles, hipStream_t st);
 
 // voxel-grid compatibility mode (pm_voxel.hip): both maps splatted into
 // [32^3][3] fixed-point grids, then their [33^3][3] summed-volume tables
@@ -217,24 +222,34 @@ struct BatchRenderScene {
   GatherMap gs, gv;
   float exposure;
   int w, h;
-  int pad;
+  int lu;            // packet gather: log2 of the march lanes per sample
   uint64_t img_off;  // first pixel of the scene's image in the batch image arena
 };
 struct BatchRenderLaunch {
   const BatchRenderScene* scenes;
-  const uint2* items;              // work items (scene, 8x8 tile), most expensive first
+  const uint2* items;              // work items (scene, tile), most expensive first
   uint32_t nitems;
   uint32_t* head;                  // work-queue counter, zero at launch
   float* rgb;                      // image arena, 3 floats per pixel
   unsigned long long* counters;    // [surface queries, volume queries]
   int heap_slots;                  // LDS heap keys per lane (>= every scene's k)
   int key_bytes;                   // heap key width: 8, 4 or 2 (gather modes 1, 2, 4)
-  int counting;                    // 1: gather mode 7 (key_bytes 2, heap_slots 64; maps with boxes and tpayload)
-  int top_levels;                  // gather mode 7: levels of each scene's trees staged in LDS per wave
+  int counting;                    // 1: the packet gather (maps with boxes and tpayload)
 };
-size_t render_batch_lds_bytes(int block_threads, int heap_slots, int key_bytes, int top_levels);
-int render_batch_occupancy(int fp64, int cone, int block_threads, int heap_slots, int key_bytes, int counting,
-                           int top_levels);  // per CU
+// Lanes of a packet-gather wave: 64 / (march lanes x samples in lanes) pixels
+// of a tile in rows, each pixel's samples, each sample's march lanes.  A tile
+// of 2^lp pixels is 8x8, 8x4, 4x4, 4x2, 2x2, 2x1 or one pixel.
+PM_HD int pk_tile_w(int lp) { return 1 << ((lp + 1) / 2); }
+PM_HD int pk_tile_h(int lp) { return 1 << (lp / 2); }
+// log2 of the march lanes per sample of a scene with volume map gv rendered in
+// a launch of `pixels` pixels, with 2^ls samples of a pixel in adjacent lanes.
+int packet_march_lanes(const RenderParams& rp, const GatherMap& gv, int ls, uint64_t pixels, int cus);
+int packet_march_lanes_batch(const RenderParams& rp, const GatherMap& gv, uint64_t pixels, int cus);
+int render_batch_occupancy(int fp64, int cone, int block_threads, int heap_slots, int key_bytes,
+                           int counting);  // workgroups per CU
+hipError_t launch_render_batch_packet(const BatchRenderLaunch& r, int fp64, int cone, int block_threads, int grid,
+                                      hipStream_t st);
+int render_batch_packet_occupancy(int fp64, int cone, int block_threads);
 hipError_t launch_tonemap(const float* rgb, size_t npix, float exposure, uchar4* out, hipStream_t st);
 hipError_t launch_gather_u32(const uint32_t* src, const uint32_t* idx, uint32_t n, uint32_t* dst, hipStream_t st);
 hipError_t launch_render_batch(const BatchRenderLaunch& r, int fp64, int cone, int block_threads, int grid,
@@ -294,18 +309,24 @@ struct CacheValueLaunch {
   GatherMap gs, gv;
   float hg_g;
   const float* in;           // query rows (9 floats)
-  const uint32_t* list;      // rows to evaluate (null: 0..n-1)
+  const uint32_t* list;      // rows to evaluate, in order (null, mode7 = 0 only: 0..n-1)
   uint32_t n;
   float* out;                // values (3 floats)
   int out_by_list;           // 1: out[list[i]], 0: out[i]
-  int mode7;                 // 1: the gather of mode 7 (k_values7), 0: the 2-byte heap gather (k_values)
-  int kind;                  // rows are 0: of either kind, 1: all surface queries, 2: all volume queries
-  uint16_t* seed_q;          // k_values7, rows with out_by_list: per record, the k-th neighbour's bucket
-                             // of its last gather (read as the counting pass's seed, then rewritten;
-                             // 0xffff: none); null: heap passes
+  int mode7;                 // 1: the packet gather (k_values_packet), 0: the 2-byte heap gather (k_values)
+  int kind;                  // 0: training rows of either kind; fallback rows: 1 all surface, 2 all volume
+  uint16_t* seed_q;          // k_values_packet: per record, the k-th neighbour's bucket of its last gather
+                             // (read as the seed, then rewritten; 0xffff: none); null: no seeds
 };
 hipError_t launch_cache_record(const CacheRecordLaunch& r, hipStream_t st);
 hipError_t launch_cache_values(const CacheValueLaunch& v, hipStream_t st);
+hipError_t launch_cache_values_packet(const CacheValueLaunch& v, hipStream_t st);
+// Row orders for the packet gather: runs of 1,024 listed rows by position, in
+// place; and order[] = all n rows by kind and position (temp: sort_rows_words
+// words).
+hipError_t launch_order_rows(const float* in, uint32_t* list, uint32_t n, hipStream_t st);
+size_t sort_rows_words(uint32_t n);
+hipError_t launch_sort_rows(const float* in, uint32_t n, uint32_t* order, uint32_t* temp, hipStream_t st);
 hipError_t launch_cache_select(const float* in, const uint32_t* list_s, uint32_t n_s, const uint32_t* list_v,
                                uint32_t n_v, uint32_t count, uint32_t seed, uint32_t frame, float* out, hipStream_t st);
 // *acc += v[0] + ... + v[n - 1] in double, in a fixed order; `part` holds

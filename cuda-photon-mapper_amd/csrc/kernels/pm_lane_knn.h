@@ -3,6 +3,7 @@
 // kernels.  Device-only; see pm_gather_lane.hip for the design notes.
 #pragma once
 
+#include "pm_estimate.h"
 #include "pm_kernels.h"
 #include "pm_wave.h"
 
@@ -223,17 +224,17 @@ struct LaneGather {
     if (m == 0) return v3(0.0f, 0.0f, 0.0f);
     float r2 = m == gs.k ? u2f(hp.h(0)) : gs.rcap2;
     float r = sqrt_(r2);
-    NSum3<float> s;
-    nsum3_init(s);
+    PowerSum s;
+    psum_init(s);
     for (int j = 0; j < m; ++j) {
       V3f pw, dir;
       load_payload_l(gs, hp.l(j), pw, dir);
       if (dot(dir, n) < 0.0f) {
         float w = CONE ? cone_weight(u2f(hp.h(j)), r) : 1.0f;
-        nsum3_add(s, pw * w);
+        psum_add(s, pw, w);
       }
     }
-    V3f sum = nsum3_get(s);
+    V3f sum = psum_get(s);
     V3f sc = v3(gs.scale[0], gs.scale[1], gs.scale[2]);
     return mul(mul(sum, albedo), sc) * surface_norm(r2, CONE);
   }
@@ -253,14 +254,15 @@ struct LaneGather {
     prev_r = m == gv.k ? sqrt_(u2f(hp.h(0))) : -1.0f;
     if (m == 0) return v3(0.0f, 0.0f, 0.0f);
     float r2 = m == gv.k ? u2f(hp.h(0)) : gv.rcap2;
-    NSum3<float> s;
-    nsum3_init(s);
+    const HgPhase ph = hg_phase(hg_g);
+    PowerSum s;
+    psum_init(s);
     for (int j = 0; j < m; ++j) {
       V3f pw, dir;
       load_payload_l(gv, hp.l(j), pw, dir);
-      nsum3_add(s, pw * phase_hg(dot(dir, wo), hg_g));
+      psum_add(s, pw, hg_eval(ph, dir, wo));
     }
-    V3f sum = nsum3_get(s);
+    V3f sum = psum_get(s);
     V3f sc = v3(gv.scale[0], gv.scale[1], gv.scale[2]);
     return mul(sum, sc) * volume_norm(r2);
   }

@@ -258,25 +258,25 @@ struct LaneGather2 {
     const GatherMap* g;
     V3f n;
     float r;
-    NSum3<float> s;
+    PowerSum s;
     __device__ void operator()(uint32_t idx, uint32_t d2) {
       V3f pw, dir;
       load_payload_l(*g, idx, pw, dir);
       if (dot(dir, n) < 0.0f) {
         float w = CONE ? cone_weight(u2f(d2), r) : 1.0f;
-        nsum3_add(s, pw * w);
+        psum_add(s, pw, w);
       }
     }
   };
   struct VolAdd {
     const GatherMap* g;
     V3f wo;
-    float hg;
-    NSum3<float> s;
+    HgPhase hg;
+    PowerSum s;
     __device__ void operator()(uint32_t idx, uint32_t) {
       V3f pw, dir;
       load_payload_l(*g, idx, pw, dir);
-      nsum3_add(s, pw * phase_hg(dot(dir, wo), hg));
+      psum_add(s, pw, hg_eval(hg, dir, wo));
     }
   };
 
@@ -293,7 +293,7 @@ struct LaneGather2 {
     const bool full = m == gs.k;
     const float r2 = full ? u2f(hp.h(0)) : gs.rcap2;
     SurfAdd add{&gs, n, sqrt_(r2), {}};
-    nsum3_init(add.s);
+    psum_init(add.s);
     SumVisitor<SurfAdd> sv{full ? hp.h(0) : caph, !full, 0u, 0u, LKEY_INF, &add};
     lane_visit(gs, x.x, x.y, x.z, sv);
     if (full) {
@@ -310,7 +310,7 @@ struct LaneGather2 {
         }
       }
     }
-    V3f sum = nsum3_get(add.s);
+    V3f sum = psum_get(add.s);
     V3f sc = v3(gs.scale[0], gs.scale[1], gs.scale[2]);
     return mul(mul(sum, albedo), sc) * surface_norm(r2, CONE);
   }
@@ -324,14 +324,14 @@ struct LaneGather2 {
       float b2 = b * b;
       if (b2 < gv.rcap2) bh = f2u(b2);
     }
-    VolAdd add{&gv, wo, hg_g, {}};
-    nsum3_init(add.s);
+    VolAdd add{&gv, wo, hg_phase(hg_g), {}};
+    psum_init(add.s);
     float r2;
     int m = knn32_gather(gv, hp, x.x, x.y, x.z, bh, caph, add, r2);
     prev_x = x;
     prev_r = m == gv.k ? sqrt_(r2) : -1.0f;
     if (m == 0) return v3(0.0f, 0.0f, 0.0f);
-    V3f sum = nsum3_get(add.s);
+    V3f sum = psum_get(add.s);
     V3f sc = v3(gv.scale[0], gv.scale[1], gv.scale[2]);
     return mul(sum, sc) * volume_norm(r2);
   }

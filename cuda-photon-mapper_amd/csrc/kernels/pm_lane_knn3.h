@@ -198,7 +198,7 @@ __device__ __forceinline__ int knn16_gather(const GatherMap& g, LaneHeap16& hp, 
   return m;
 }
 
-template <bool CONE, int NB = 8>
+template <bool CONE, int NB = 8, class P = SumFp64>
 struct LaneGather3 {
   GatherMap gs, gv;
   LaneHeap16 hp;
@@ -212,25 +212,25 @@ struct LaneGather3 {
   struct SurfAdd {
     const GatherMap* g;
     V3f n;
-    NSum3<float> s0, s1;
+    PowerSum s0, s1;
     __device__ void operator()(uint32_t idx, uint32_t d2) {
       V3f pw, dir;
       load_payload_l(*g, idx, pw, dir);
       if (dot(dir, n) < 0.0f) {
-        nsum3_add(s0, pw);
-        if (CONE) nsum3_add(s1, pw * sqrt_(u2f(d2)));
+        psum_add(s0, pw);
+        if (CONE) psum_add(s1, pw, sqrt_(u2f(d2)));
       }
     }
   };
   struct VolAdd {
     const GatherMap* g;
     V3f wo;
-    float hg;
-    NSum3<float> s;
+    typename P::Phase hg;
+    PowerSum s;
     __device__ void operator()(uint32_t idx, uint32_t) {
       V3f pw, dir;
       load_payload_l(*g, idx, pw, dir);
-      nsum3_add(s, pw * phase_hg(dot(dir, wo), hg));
+      P::add(s, pw, dir, wo, hg);
     }
   };
 
@@ -240,13 +240,13 @@ struct LaneGather3 {
     SurfAdd add;
     add.g = &gs;
     add.n = n;
-    nsum3_init(add.s0);
-    nsum3_init(add.s1);
+    psum_init(add.s0);
+    psum_init(add.s1);
     float r2;
     int m = knn16_gather<NB>(gs, hp, x.x, x.y, x.z, caph, caph, add, r2);
     if (m == 0) return v3(0.0f, 0.0f, 0.0f);
-    V3f sum = nsum3_get(add.s0);
-    if (CONE) sum = sum - nsum3_get(add.s1) * (1.0f / (1.1f * sqrt_(r2)));
+    V3f sum = psum_get(add.s0);
+    if (CONE) sum = sum - psum_get(add.s1) * (1.0f / (1.1f * sqrt_(r2)));
     V3f sc = v3(gs.scale[0], gs.scale[1], gs.scale[2]);
     return mul(mul(sum, albedo), sc) * surface_norm(r2, CONE);
   }
@@ -260,14 +260,14 @@ struct LaneGather3 {
       float b2 = b * b;
       if (b2 < gv.rcap2) bh = f2u(b2);
     }
-    VolAdd add{&gv, wo, hg_g, {}};
-    nsum3_init(add.s);
+    VolAdd add{&gv, wo, P::phase(hg_g), {}};
+    psum_init(add.s);
     float r2;
     int m = knn16_gather<NB>(gv, hp, x.x, x.y, x.z, bh, caph, add, r2);
     prev_x = x;
     prev_r = m == gv.k ? sqrt_(r2) : -1.0f;
     if (m == 0) return v3(0.0f, 0.0f, 0.0f);
-    V3f sum = nsum3_get(add.s);
+    V3f sum = psum_get(add.s);
     V3f sc = v3(gv.scale[0], gv.scale[1], gv.scale[2]);
     return mul(sum, sc) * volume_norm(r2);
   }

@@ -1,0 +1,96 @@
+"""The packet gather (gather mode 7) at the sizes where its stages, windows,
+groups and tie handling change, on caller-given photon maps, against the
+8-byte heap gather (mode 1), which keeps exact (d^2, index) keys and shares
+none of that code.  Both sum a query's neighbours in FP64, so a query's FP32
+sum differs by at most its last bit between them, and a pixel's radiance (a
+sum of non-negative terms, each off by at most 2^-23 of itself, and the
+rounding of the sums) by less than 5e-7 of itself.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+import pmamd
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 5e-7
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def volume_points(rng, layout, n):
+    if layout == "uniform":
+        return rng.random((n, 3), dtype=np.float32)
+    if layout == "coincident":  # 50 photons at each place: counters wrap, ties go by index
+        return np.repeat(rng.random((n // 50, 3), dtype=np.float32), 50, axis=0)
+    if layout == "lattice":  # many equal distances
+        m = int(round(n ** (1.0 / 3.0)))
+        g = (np.indices((m, m, m)).reshape(3, -1).T + 0.5) / m
+        return g.astype(np.float32)
+    # nine in ten inside a small ball in view: stages overflow, groups split
+    p = rng.random((n, 3), dtype=np.float32)
+    d = rng.normal(size=(n, 3))
+    ball = 0.5 + 0.02 * d / np.linalg.norm(d, axis=1, keepdims=True) * rng.random((n, 1)) ** (1.0 / 3.0)
+    inside = np.arange(n) % 10 != 0
+    p[inside] = ball[inside].astype(np.float32)
+    return p
+
+
+def wall_points(rng, layout, n):
+    p = volume_points(rng, layout, n)
+    w = np.arange(len(p)) % 5
+    p[np.arange(len(p)), np.array([0, 0, 1, 1, 2])[w]] = np.array([0, 1, 0, 1, 1], np.float32)[w]
+    return p
+
+
+CASES = [
+    # layout, photons, leaf, k, cap, spp, width, height, spheres
+    ("uniform", 1, 32, 32, 0.05, 1, 33, 17, 2),
+    ("uniform", 64, 64, 64, 3.0, 1, 9, 7, 2),  # exactly k points, one leaf, all in reach
+    ("uniform", 65, 64, 64, 3.0, 1, 9, 7, 2),
+    ("uniform", 5000, 1, 1, 0.05, 1, 40, 24, 2),
+    ("uniform", 5001, 7, 33, 0.2, 3, 24, 16, 2),
+    ("uniform", 40000, 52, 64, 0.5, 4, 24, 16, 2),
+    ("uniform", 40000, 64, 64, 0.03, 16, 7, 5, 2),
+    ("uniform", 200000, 32, 32, 0.05, 2, 19, 11, 200),  # queries far apart: many groups
+    ("coincident", 20000, 32, 32, 0.2, 1, 24, 16, 2),
+    ("coincident", 20000, 16, 64, 0.2, 4, 12, 8, 2),
+    ("lattice", 27000, 32, 64, 0.2, 1, 24, 16, 2),
+    ("dense", 200000, 52, 64, 0.1, 4, 24, 16, 2),
+    ("dense", 200000, 8, 64, 0.5, 1, 24, 16, 2),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c[:7]))
+def test_packet_equals_heap_gather(case):
+    layout, n, leaf, k, cap, spp, w, h, spheres = case
+    say("case: packet gather, %s, n=%d, leaf=%d, k=%d, r<=%g, %dx%dx%d" % (layout, n, leaf, k, cap, w, h, spp))
+    c = pmamd.batch_scene(3, 5) if spheres > 2 else pmamd.preset(1)
+    c.leaf_size = leaf
+    c.k_surface = c.k_volume = k
+    c.rcap_surface = c.rcap_volume = cap
+    c.width, c.height, c.spp = w, h, spp
+    c.medium, c.sigma_s, c.sigma_a, c.hg_g = pmamd.PM_MEDIUM_HOMOGENEOUS, 0.1, 0.01, 0.6
+    rng = np.random.default_rng(11)
+    g = pmamd.PhotonMapper(c)
+    for which, pos in ((pmamd.PM_MAP_SURFACE, wall_points(rng, layout, n)),
+                       (pmamd.PM_MAP_VOLUME, volume_points(rng, layout, n))):
+        d = rng.normal(size=pos.shape)
+        d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+        g.set_records(which, pos, rng.uniform(0.5, 1.5, pos.shape).astype(np.float32), d, 2 * n)
+    g.build()
+    g.set_option(pmamd.PM_OPT_GATHER_MODE, 1)
+    ref = g.render()
+    rq = g.stats()
+    g.set_option(pmamd.PM_OPT_GATHER_MODE, 7)
+    img = g.render()
+    q = g.stats()
+    assert (q.surface_queries, q.volume_queries) == (rq.surface_queries, rq.volume_queries)
+    assert q.volume_queries > 0 and (n < 100 or ref.max() > 0)
+    np.testing.assert_allclose(img, ref, rtol=RTOL, atol=0)
+    g.close()
