@@ -596,7 +596,7 @@ def main():
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": (tr.get("bytes_per_launch") if tr else None),
-            "kernel": "k_render_lane7s (eye ray + march + kNN gather, a pixel's samples in adjacent lanes)",
+            "kernel": "k_render_packet (eye ray + march + kNN gather, one search for a wave's queries)",
             "bytes_per_query": bpq,
             "queries_per_launch": int(q_frame), "kernel_ms": round(kern_ms, 3)}
     if vp:

@@ -13,7 +13,7 @@
 //                       k_values otherwise) and trains the MLP (pm_mlp.hip);
 //                       each batch's pre-update errors are binned into a
 //                       16^3 x {surface, volume} grid (by the fused forward
-//                       pass, k_fwd_fused in pm_mlp_train.hip)
+//                       pass, k_fwd_bwd in pm_mlp_train.hip)
 //   5. inference      : MLP over the volume records (all records when surface
 //                       records are cached too; pm_mlp_infer.hip)
 //   6. fallback       : records in cells whose mean training error exceeds

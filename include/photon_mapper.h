@@ -193,14 +193,13 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                          the exact order restored inside the k-th bucket,
  *                          leaf points loaded 4 at a time under a
  *                          5-waves-per-SIMD register budget,
- *                      5 = auto (default): 7 when the frame has at least 16
- *                          8x8 tiles per compute unit and the maps hold at
- *                          least 2^20 records, else 1;
- *                      7 = as 4, with each march step's second pass merged
- *                          into the next step's first-pass traversal and the
- *                          first passes done by counting in a window of 256
- *                          buckets around the previous step's
- *                          k-th-neighbour bucket (heap pass on a miss);
+ *                      5 = auto (default): as 7;
+ *                      7 = one search of the kd-tree for the 64 queries of a
+ *                          wave (the packet gather): the points near the
+ *                          queries' box staged in LDS, each query's k-th
+ *                          distance found by counting in a window of 128
+ *                          buckets of d^2 (2^-7 wide) around the bucket of
+ *                          its previous march step, then summed up to it;
  *                      (3 and 6 are not used: PM_ERR_INVALID);
  *                      every mode gives the same neighbour sets and images;
  * PM_OPT_BLOCKS_PER_CU workgroups per compute unit of the persistent mode-0 grid;
@@ -216,15 +215,15 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                      14..20 (default 20): smaller chunks keep the layer-1
  *                      activations in the on-die caches between the two launches,
  *                      larger ones launch fewer, fuller grids (faster at 1080p);
- * PM_OPT_TILE_REGIONS  order in which the lane modes' workgroups take 8x8 tiles:
+ * PM_OPT_TILE_REGIONS  order in which the lane and packet modes' workgroups take tiles:
  *                      0 = raster order (default), rx = 1, 2, 4 or 8 = the
  *                      frame cut into rx x (8 / rx) regions, one per XCD
  *                      (workgroups go to the 8 XCDs round-robin), so that each
  *                      XCD's L2 serves one compact part of the frame;
  * PM_OPT_SAMPLE_LANES  gather mode 7 with spp = 2, 4, 8 or 16: 1 = the samples of a
- *                      pixel in adjacent lanes (default; a wave renders 64 / spp
- *                      pixels in raster tile order), 0 = one lane loops over a
- *                      pixel's samples (PM_OPT_TILE_REGIONS applies to this form);
+ *                      pixel in adjacent lanes (default; raster tile order),
+ *                      0 = the wave loops over its pixels' samples
+ *                      (PM_OPT_TILE_REGIONS applies to this form);
  * PM_OPT_RENDER_MEDIA  1 = pm_render / pm_render_crop / pm_render_cache_crop
  *                      march the medium (default, when the scene has one),
  *                      0 = they gather at surface hits only: the surface-gather
@@ -242,12 +241,11 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  * PM_OPT_CACHE_SEEDS   1 = the cache render's exact fallback (gather modes 7
  *                      and auto) starts each record from its k-th neighbour's
  *                      bucket of the previous call while the records and the
- *                      photon positions are unchanged (default), 0 = heap
- *                      passes every call; the values are the same bits;
- * PM_OPT_TOP_LEVELS    gather mode 7 (also when auto picks it): the top 0..7
- *                      levels of both kd-trees (2^levels - 1 nodes, 48 B each)
- *                      staged in each wave's LDS for the traversals to read,
- *                      0 = none (default), every node read from HBM;
+ *                      photon positions are unchanged (default), 0 = unseeded
+ *                      searches every call; the values are the same bits;
+ * PM_OPT_TOP_LEVELS    0..7, default 0: accepted, without effect (the packet
+ *                      gather of mode 7 reads 64 nodes a step, so that no
+ *                      top of the tree needs to be kept in LDS);
  * PM_OPT_VOXEL_GRID    0 = the k-NN estimate (default); 1 = the reference's
  *                      voxel-grid estimate (photonMappingKernel.cu:314-389,
  *                      :831-870): both maps splatted into 32^3 grids over the
@@ -356,10 +354,9 @@ typedef struct pm_batch_tuning {
   int block_threads;  /* render workgroup size: 64, 128, 192 or 256 */
   int heap_slots;     /* LDS heap keys per lane: 32 or 64 (>= every scene's k) */
   int heap_key_bytes; /* heap key width: 8 (d^2, index), 4 (d^2) or 2 (d^2 bucket); see PM_OPT_GATHER_MODE */
-  int gather_mode;    /* 0: the heap gather of heap_key_bytes (modes 1, 2, 4); 7: gather mode 7, which needs
-                         heap_key_bytes 2 and heap_slots 64 (its bucket counters take that LDS) */
-  int top_levels;     /* LDS tile, gather mode 7 only: the top 0..7 levels of the current scene's two kd-trees
-                         (2^levels - 1 nodes each, 48 B per node) staged in each wave's LDS, 0 = none */
+  int gather_mode;    /* 0: the heap gather of heap_key_bytes (modes 1, 2, 4); 7: gather mode 7, which the
+                         packet gather, set with heap_key_bytes 2 and heap_slots 64 (default) */
+  int top_levels;     /* 0..7 (only 0 without gather mode 7): accepted, without effect */
 } pm_batch_tuning;
 
 typedef struct pm_batch_stats {
@@ -388,8 +385,7 @@ int pm_batch_set_tuning(pm_batch* b, const pm_batch_tuning* t);
 /* Times the kd-build and a 1-in-`sample_stride` subset of the render work
  * items for a staged sweep: heap key width {8, 4, 2} x heap slots {32 (when
  * every k <= 32), 64} and gather mode 7, then leaf size {4, 8, 16, 32}, then
- * workgroup size {64, 128, 256}, then (when gather mode 7 won) the LDS tile
- * top_levels {0, 3, 5, 7}, each stage from the best so far; keeps the
+ * workgroup size {64, 128, 256}, each stage from the best so far; keeps the
  * fastest and returns it (and its time). */
 int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out, double* best_ms_out);
 /* One frame of every scene (one graph launch); blocking. */
