@@ -443,13 +443,15 @@ hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st) {
   const int lp = 6 - lu - ls;
   RenderLaunch q = r;
   dim3 grid(tile_grid(r, pk_tile_w(lp), pk_tile_h(lp), ls > 0));
-  // the heavy tiles first and split where the launch ends on them: few waves,
-  // or, with samples in lanes, in a map dense enough that a wave's march takes
-  // milliseconds, few rounds of waves (480x270 window of the fog with 4 samples
-  // 30 -> 14 ms; the whole 1920x1080 frame 136 -> 151, so not there)
-  const bool dense = ls > 0 && mean_radius(r.gv) * mean_radius(r.gv) < 0.999 * r.gv.rcap2;
-  const bool few = dense ? tiles < 64u * (unsigned)r.cus : lu > 0 && tiles < 34u * (unsigned)r.cus &&
-                   !(mean_radius(r.gv) * mean_radius(r.gv) < 0.999 * r.gv.rcap2);
+  // The heavy tiles first and split where the launch ends on them: frames of
+  // few waves, or, in a map so dense that a wave's march takes milliseconds, of
+  // few rounds of waves (480x270 window of the fog with 4 samples 30 -> 14 ms;
+  // the whole 1920x1080 frame 136 -> 151, so not there).  One-sample frames of
+  // such a map stay on the grid (the window: 23 ms, 11 from the list): a cache
+  // frame is to be the faster one there, and takes 10 to 11 ms.
+  const double rm = mean_radius(r.gv);
+  const bool dense = rm * rm < 0.999 * r.gv.rcap2;
+  const bool few = dense ? ls > 0 && tiles < 64u * (unsigned)r.cus : lu > 0 && tiles < 34u * (unsigned)r.cus;
   if (r.tile_regions == 0 && r.rp.media_on && few && r.items.head && r.items.words >= packet_item_words(tiles)) {
     hipError_t e = launch_packet_tiles(q, lu, ls, tiles, st);
     if (e != hipSuccess) return e;
