@@ -67,10 +67,6 @@ __device__ __forceinline__ void pk_sync() {
 __device__ __forceinline__ uint32_t pk_rank(uint64_t m) {  // set bits of m below this lane
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
-// v + 1 in the lanes of m: one add with carry-in (a select and an add otherwise).
-__device__ __forceinline__ void pk_inc(uint32_t& v, uint64_t m) {
-  asm("v_addc_co_u32_e64 %0, vcc, 0, %0, %1" : "+v"(v) : "s"(m) : "vcc");
-}
 template <int CTRL>
 __device__ __forceinline__ uint32_t pk_dpp(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false);
@@ -518,9 +514,9 @@ __device__ __forceinline__ void packet_gather(const GatherMap& g, PacketLds& S, 
             if (c0 + j >= m) break;
             const uint32_t d = f2u(dist2(q.x, q.y, q.z, p[j].x, p[j].y, p[j].z));
             const uint32_t t = d - base;
-            pk_inc(below, ballot(d < base));
+            below += d < base ? 1u : 0u;
             const bool in = t < width;
-            pk_inc(inwin, ballot(in));
+            inwin += in ? 1u : 0u;
             if (in)
               __hip_atomic_fetch_add(&S.cnt[(t >> 19) * 64u + (uint32_t)lane], 1u << ((t >> 14) & 28u),
                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
