@@ -62,8 +62,10 @@ __device__ __forceinline__ V3f psum_get(const PowerSum& s) { return v3((float)s.
 // g.  den^(-3/2) from the hardware reciprocal square root (1 ulp) and two
 // products: within 4e-7 of the closed form on the FP32 den, against 6e-7 for
 // the Newton steps of phase_hg (core/pm_scene.h), and 10 instructions fewer.
-// |g| < 1 gives den >= 2^-48; the clamp keeps directions that are not quite
-// of unit length from reaching 0.
+// |g| < 1 gives den >= 2^-48 for directions of unit length.  A longer one (BF16
+// storage rounds each component to 2^-9, and callers give their own) can take
+// den below 0: such a photon has no weight, as in phase_hg, whose Newton steps
+// underflow there (down to -0.2).
 struct HgPhase {
   float a, b, c;  // 1 + g^2, -2 g, (1 - g^2) / (4 pi)
 };
@@ -72,9 +74,9 @@ __device__ __forceinline__ HgPhase hg_phase(float g) {
 }
 __device__ __forceinline__ float hg_eval(const HgPhase& h, V3f dir, V3f wo) {
   const float cs = __builtin_fmaf(dir.z, wo.z, __builtin_fmaf(dir.y, wo.y, dir.x * wo.x));
-  const float den = __builtin_fmaxf(__builtin_fmaf(h.b, cs, h.a), 3.5527137e-15f);
+  const float den = __builtin_fmaf(h.b, cs, h.a);
   const float y = __builtin_amdgcn_rsqf(den);
-  return h.c * ((y * y) * y);
+  return den < 0.0f ? 0.0f : h.c * ((y * y) * y);
 }
 
 // The two kinds of terms a gather sums.  SumFp64: the renders and the cache's

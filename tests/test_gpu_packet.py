@@ -94,3 +94,28 @@ def test_packet_equals_heap_gather(case):
     assert q.volume_queries > 0 and (n < 100 or ref.max() > 0)
     np.testing.assert_allclose(img, ref, rtol=RTOL, atol=0)
     g.close()
+
+
+@pytest.mark.parametrize("storage", [pmamd.PM_STORE_FP32, pmamd.PM_STORE_BF16])
+@pytest.mark.parametrize("mode", [0, 1, 2, 4, 7])
+def test_directions_longer_than_one_have_no_weight(mode, storage):
+    """At g = 0.99 a photon that travels 1.05 long along the view direction has
+    1 + g^2 - 2 g cos = -0.1: no phase function, and no weight in the sum.  A
+    view that meets no other photons is black."""
+    say("case: directions of length 1.05, g = 0.99, gather mode %d, storage %d" % (mode, storage))
+    c = pmamd.preset(1)
+    c.n_spheres = 0
+    c.width, c.height, c.focal, c.storage = 8, 8, 50.0, storage
+    c.medium, c.sigma_s, c.sigma_a, c.hg_g = pmamd.PM_MEDIUM_HOMOGENEOUS, 0.1, 0.01, 0.99
+    rng = np.random.default_rng(3)
+    pos = rng.random((20000, 3), dtype=np.float32)
+    none = np.zeros((0, 3), np.float32)
+    g = pmamd.PhotonMapper(c)
+    g.set_records(pmamd.PM_MAP_SURFACE, none, none, none, 1)
+    g.set_records(pmamd.PM_MAP_VOLUME, pos, np.ones_like(pos), np.tile(np.float32([0, 0, -1.05]), (len(pos), 1)), 1)
+    g.build()
+    g.set_option(pmamd.PM_OPT_GATHER_MODE, mode)
+    img = g.render()
+    assert g.stats().volume_queries > 0
+    assert np.array_equal(img, np.zeros_like(img)), img.max()
+    g.close()
