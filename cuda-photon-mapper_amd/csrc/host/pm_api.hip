@@ -516,14 +516,11 @@ int render_crop_impl(pm_context* c, int x0, int y0, int w, int h, float* rgb_dev
     HIPCHK(launch_render_voxel(r, G, c->stream));
   } else {
   HIPCHK(hipEventRecord(c->e0, c->stream));
+  if (r.gather_mode == 5) r.gather_mode = packet_pays(r) ? 7 : 1;
   switch (r.gather_mode) {
     case 0: HIPCHK(launch_render(r, c->stream)); break;
     case 1: HIPCHK(launch_render_lane(r, c->stream)); break;
     case 4: HIPCHK(launch_render_lane4(r, c->stream)); break;
-    // auto: the packet gather, the fastest at every size (one GPU, ms, against
-    // the 8-byte heap: 64x48 room crop 0.4 / 6.1, 256x256 room 3.1 / 14, 477x271x4
-    // fog crop 34 / 467)
-    case 5:
     case 7:
       // the work items' scratch: grown here, or as pm_build left it for the
       // caller that allocates nothing (a larger frame then renders in raster order)

@@ -608,6 +608,36 @@ int apply_tuning(pm_batch* b, const pm_batch_tuning& t, bool capture_graph) {
   return capture(b);
 }
 
+// The packet gather where it pays for most of the batch's samples, else the
+// 2-byte heap.
+pm_batch_tuning default_tuning(const pm_batch* b) {
+  double packet = 0.0, heap = 0.0;
+  for (int s = 0; s < b->ns; ++s) {
+    const pm_config& c = b->cfg[s];
+    const RenderParams rp = render_params(c);
+    GatherMap gs, gv;
+    memset(&gs, 0, sizeof(gs));
+    memset(&gv, 0, sizeof(gv));
+    gs.n = b->nrec_s[s];
+    gs.k = c.k_surface;
+    gs.rcap2 = c.rcap_surface * c.rcap_surface;
+    gv.n = b->nrec_v[s];
+    gv.k = c.k_volume;
+    gv.rcap2 = c.rcap_volume * c.rcap_volume;
+    const bool pays =
+        packet_pays(rp, rp.media_on != 0, gs, gv, 0, batch_march_lanes(b, s), b->npix, b->cus);
+    (pays ? packet : heap) += (double)c.width * (double)c.height * (double)c.spp;
+  }
+  pm_batch_tuning t;
+  t.leaf_size = 32;
+  t.block_threads = 64;
+  t.gather_mode = packet >= heap ? 7 : 0;
+  t.heap_slots = t.gather_mode == 7 || b->kmax > 32 ? 64 : 32;
+  t.heap_key_bytes = 2;
+  t.top_levels = 0;
+  return t;
+}
+
 void destroy(pm_batch* b) {
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   release_graph(b);
@@ -689,17 +719,10 @@ int pm_batch_create(const pm_config* cfgs, int n, pm_batch** out) {
     return PM_ERR_HIP;
   }
   const auto t0 = std::chrono::steady_clock::now();
-  pm_batch_tuning t;
-  t.leaf_size = 32;
-  t.block_threads = 64;
-  t.heap_slots = 64;
-  t.heap_key_bytes = 2;
-  t.gather_mode = 7;
-  t.top_levels = 0;
   int r = setup_scenes(b);
   if (r == PM_OK) r = size_records(b);
   if (r == PM_OK) r = setup_render(b);
-  if (r == PM_OK) r = apply_tuning(b, t, true);
+  if (r == PM_OK) r = apply_tuning(b, default_tuning(b), true);
   if (r != PM_OK) {
     destroy(b);
     return r;

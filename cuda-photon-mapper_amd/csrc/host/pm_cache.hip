@@ -413,8 +413,10 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   HIPCHK(c->small.ensure(64));
   unsigned long long* ntot_dev = (unsigned long long*)(c->small.as<uint32_t>() + 14);
   HIPCHK(launch_count_total(k.rec_cnt.as<uint32_t>(), npix, ntot_dev, st));
-  // exact values with the gather of mode 7 under modes 7 and 5 (auto)
-  const int mode7 = c->gather_mode == 7 || c->gather_mode == 5 ? 1 : 0;
+  // exact values with the gather of mode 7, under mode 5 (auto) where it pays
+  GatherMap gs = make_gather_map(c, c->ms.m, c->cfg.k_surface, c->cfg.rcap_surface);
+  GatherMap gv = make_gather_map(c, c->mv.m, c->cfg.k_volume, c->cfg.rcap_volume);
+  const int mode7 = c->gather_mode == 7 || (c->gather_mode == 5 && packet_pays_rows(gv)) ? 1 : 0;
   uint64_t N = 0;
   unsigned long long hh[2] = {0ull, 0ull};  // the maps' fingerprints (prepare_seeds), in the same read-back
   HIPCHK(hipMemcpyAsync(&N, ntot_dev, 8, hipMemcpyDeviceToHost, st));
@@ -439,8 +441,6 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   HIPCHK(launch_cache_record(rl, st));
   HIPCHK(hipEventRecord(ev[1], st));
   // 4: online training on a subset with exact kNN targets
-  GatherMap gs = make_gather_map(c, c->ms.m, c->cfg.k_surface, c->cfg.rcap_surface);
-  GatherMap gv = make_gather_map(c, c->mv.m, c->cfg.k_volume, c->cfg.rcap_volume);
   const uint32_t ncell = 2u * CACHE_GRID * CACHE_GRID * CACHE_GRID;
   HIPCHK(k.err_sum.ensure(8ull * ncell));
   HIPCHK(k.err_cnt.ensure(4ull * ncell));

@@ -185,6 +185,12 @@ hipError_t launch_render_lane(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_lane2(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_lane4(const RenderLaunch& r, hipStream_t st);
 hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st);
+// Whether auto renders r, a batch's default a scene, and auto a cache frame's
+// exact values, with the packet gather (else with a heap).
+bool packet_pays(const RenderLaunch& r);
+bool packet_pays(const RenderParams& rp, bool march, const GatherMap& gs, const GatherMap& gv, int ls, int lu,
+                 uint64_t pixels, int cus);
+bool packet_pays_rows(const GatherMap& gv);
 // Tiles of a packet render of r, and the lists of its heavy and light items
 // into r.items (head set, packet_item_words(tiles) words).
 uint32_t packet_tiles(const RenderLaunch& r);

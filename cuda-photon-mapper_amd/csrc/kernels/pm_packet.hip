@@ -411,14 +411,86 @@ int packet_march_lanes_batch(const RenderParams& rp, const GatherMap& gv, uint64
 
 size_t packet_item_words(uint32_t tiles) { return 4 + 5ull * tiles; }
 
+// log2 of the samples of a pixel that go to adjacent lanes.
+static int packet_sample_lanes(const RenderLaunch& r) {
+  const int spp = r.rp.spp;
+  const int ls = r.sample_lanes && (spp == 2 || spp == 4 || spp == 8 || spp == 16) ? __builtin_ctz((unsigned)spp) : 0;
+  // a launch holds fewer than 2^32 lanes
+  return (((uint64_t)r.w + 7) * ((uint64_t)r.h + 7)) << ls >= 1ull << 31 ? 0 : ls;
+}
+
+// Whether the packet gather renders a scene faster than the 8-byte heap of mode
+// 1 (its 2-byte form in a batch): ls and lu are the log2 of its sample and march
+// lanes, pixels those of the launch.  Searches are shared, so the packet gather
+// loses where a wave's balls do not overlap: each of its 64 queries is then a
+// search of its own, 64 in a row.
+//
+// With a march, a wave's points are spread over a march step along their rays
+// (the samples' offsets), so balls of about a step or less in which hardly any
+// photon lies go to the heap, unless the launch is so small that eight march
+// lanes split its chains; fewer photons are enough where four samples or more
+// lie together in lanes, and one neighbour's ball counts in place of the cap.
+// 256x256 room, 2,452 to 718,541 records, r <= 0.005, k = 1 to 64: heap 1.2 to
+// 4.3 ms, packet 16 to 22; r <= 0.02: 1.4 to 9.5 and 1.1 to 3.9 (k = 1: 9.7);
+// 640x360 with 4 samples, r <= 0.05: 10 to 180 and 2 to 14.
+//
+// Without one, a wave makes one search, without a seed.  Four or more samples
+// in lanes pay for it (640x360x4, k = 32, r <= 0.05: heap 1.1 to 5.2 ms, packet
+// 0.5 to 1.8) unless the cap is so much wider than the ball that the first
+// bound is loose (k = 8, r <= 0.47, a ball of a quarter tile: 1.5 and 4.5).
+// Otherwise full balls, of 13 neighbours or more, pay where the cap is not far
+// beyond them (718,541 records, 640x360, k = 32: 1.3 and 0.7 at r <= 0.02, 1.3
+// and 3.7 at r <= 0.15) and the launch is of less than a wave per CU, or of
+// many, or its balls are as wide as four tiles (48,578 records, r <= 0.05,
+// 3,600 waves, 1.5 tiles: 0.8 and 1.6); and emptier ones if wider than five.
+//
+// Over 4,800 random frames (scene, photons, k, cap, size, samples) the choice
+// takes 1.017 times the faster one's time with a march (the packet gather
+// always: 1.05, and up to 11 times the heap's) and 1.07 without (1.33, up to 31).
+bool packet_pays(const RenderParams& rp, bool march, const GatherMap& gs, const GatherMap& gv, int ls, int lu,
+                 uint64_t pixels, int cus) {
+  const uint64_t waves = (pixels << ls) >> 6, cu = (uint64_t)cus;  // without march lanes
+  const GatherMap& g = march ? gv : gs;
+  const double cap2 = (double)g.rcap2, cap = sqrt(cap2), n = (double)g.n, k = (double)g.k;
+  if (march) {
+    if (lu >= 3) return true;
+    const double step = (double)rp.march_step, in_cap = 4.2 * n * cap2 * cap;
+    const double ball = in_cap > 1.0 ? cap / cbrt(in_cap) : cap;  // one neighbour's
+    if (g.k == 1 && ls < 2 && ball < 1.7 * step) return false;
+    return cap >= 1.2 * step || in_cap >= (ls < 2 ? 0.3 : 0.002);
+  }
+  constexpr double kWalls = 5.0;                   // area of the room's five walls
+  const double in_cap = 3.14 * n * cap2 / kWalls;  // photons within the cap of a hit
+  const double tile = (double)pk_tile_w(6 - ls) / ((double)rp.focal * (double)rp.height);  // at distance 1
+  const double tiles = cap * (in_cap > k ? sqrt(k / in_cap) : 1.0) / tile;                 // a ball's radius
+  if (ls >= 2) return in_cap <= 5000.0 || tiles >= 0.4;
+  if (std::min(in_cap, k) >= 13.0)
+    return in_cap <= 1500.0 && (waves <= cu || (in_cap >= 45.0 && (waves >= 16u * cu || tiles >= 4.0)));
+  return tiles >= 5.4 && waves < 32u * cu;
+}
+
+// The same for the exact values of a cache frame's records, in the volume map:
+// listed rows are further apart than a tile's march points, so it is only
+// whether a photon or none is near.  64x48 to 640x360 frames with all records
+// gathered, packet over heap (2-byte keys) time of the frame, medians: fewer
+// than 0.001 photons within the cap 1.8 to 2.6, 0.01 to 0.1 1.1 to 1.8, 0.1 to 1
+// 0.7 to 1.1 (at caps of a step and more), more 0.4 to 0.7.
+bool packet_pays_rows(const GatherMap& gv) {
+  return 4.2 * (double)gv.n * (double)gv.rcap2 * sqrt((double)gv.rcap2) >= 0.1;
+}
+
 // The launch's lane layout and tile count.
 static uint32_t packet_layout(const RenderLaunch& r, int& lu, int& ls) {
-  const int spp = r.rp.spp;
-  ls = r.sample_lanes && (spp == 2 || spp == 4 || spp == 8 || spp == 16) ? __builtin_ctz((unsigned)spp) : 0;
-  if ((((uint64_t)r.w + 7) * ((uint64_t)r.h + 7)) << ls >= 1ull << 31) ls = 0;  // a launch holds fewer than 2^32 lanes
+  ls = packet_sample_lanes(r);
   lu = packet_march_lanes(r.rp, r.gv, ls, (uint64_t)r.w * (uint64_t)r.h, r.cus);
   const int lp = 6 - lu - ls;
   return (uint32_t)((r.w + pk_tile_w(lp) - 1) / pk_tile_w(lp)) * (uint32_t)((r.h + pk_tile_h(lp) - 1) / pk_tile_h(lp));
+}
+
+bool packet_pays(const RenderLaunch& r) {
+  int lu, ls;
+  packet_layout(r, lu, ls);
+  return packet_pays(r.rp, r.rp.media_on != 0, r.gs, r.gv, ls, lu, (uint64_t)r.w * (uint64_t)r.h, r.cus);
 }
 
 uint32_t packet_tiles(const RenderLaunch& r) {

@@ -193,7 +193,13 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                          the exact order restored inside the k-th bucket,
  *                          leaf points loaded 4 at a time under a
  *                          5-waves-per-SIMD register budget,
- *                      5 = auto (default): as 7;
+ *                      5 = auto (default): 7, or 1 where the neighbour balls
+ *                          of a wave's queries would not overlap (caps below a
+ *                          march step in nearly empty maps, and surface hits
+ *                          alone with fewer than 4 samples in lanes, unless
+ *                          their balls are full); the cache render's exact
+ *                          values: 7, or the heap of mode 4 where hardly any
+ *                          point has a photon within the cap;
  *                      7 = one search of the kd-tree for the 64 queries of a
  *                          wave (the packet gather): the points near the
  *                          queries' box staged in LDS, each query's k-th
@@ -354,8 +360,9 @@ typedef struct pm_batch_tuning {
   int block_threads;  /* render workgroup size: 64, 128, 192 or 256 */
   int heap_slots;     /* LDS heap keys per lane: 32 or 64 (>= every scene's k) */
   int heap_key_bytes; /* heap key width: 8 (d^2, index), 4 (d^2) or 2 (d^2 bucket); see PM_OPT_GATHER_MODE */
-  int gather_mode;    /* 0: the heap gather of heap_key_bytes (modes 1, 2, 4); 7: gather mode 7, which the
-                         packet gather, set with heap_key_bytes 2 and heap_slots 64 (default) */
+  int gather_mode;    /* 0: the heap gather of heap_key_bytes (modes 1, 2, 4); 7: the packet gather of mode 7, set
+                         with heap_key_bytes 2 and heap_slots 64.  Default: 7 where auto would take it for most of the
+                         batch's samples, else 0 with 2-byte keys */
   int top_levels;     /* 0..7 (only 0 without gather mode 7): accepted, without effect */
 } pm_batch_tuning;
 

@@ -119,3 +119,89 @@ def test_directions_longer_than_one_have_no_weight(mode, storage):
     assert g.stats().volume_queries > 0
     assert np.array_equal(img, np.zeros_like(img)), img.max()
     g.close()
+
+
+# photons, k, cap, width, height, spp, march; the faster gather is 2 to 12 times the other
+AUTO_CASES = [
+    (1000, 32, 0.005, 256, 256, 1, 1),    # balls below a march step in an empty map: heap
+    (20000, 8, 0.004, 440, 220, 1, 1),
+    (20000, 32, 0.05, 64, 48, 1, 1),      # few waves: packet, march steps in lanes
+    (100000, 32, 0.05, 256, 256, 1, 1),
+    (20000, 4, 0.15, 640, 360, 4, 1),
+    (20000, 32, 0.05, 640, 360, 1, 0),    # surface hits: a search per wave and no seed
+    (100000, 32, 0.02, 960, 540, 1, 0),   # full balls, the cap close to them
+    (100000, 16, 0.4, 200, 150, 1, 0),
+    (100000, 1, 0.1, 256, 256, 1, 0),
+    (100000, 64, 0.03, 640, 360, 4, 0),   # samples in lanes
+]
+
+
+@pytest.mark.parametrize("case", AUTO_CASES, ids=lambda c: "-".join(str(v) for v in c))
+def test_auto_takes_the_faster_gather(case):
+    photons, k, cap, w, h, spp, march = case
+    say("case: gather mode of auto, %d photons, k=%d, r<=%g, %dx%dx%d, march %d" % case)
+    c = pmamd.preset(1)
+    c.n_emit, c.k_surface, c.k_volume, c.rcap_surface, c.rcap_volume = photons, k, k, cap, cap
+    c.width, c.height, c.spp = w, h, spp
+    g = pmamd.PhotonMapper(c)
+    g.emit()
+    g.build()
+    g.set_option(pmamd.PM_OPT_RENDER_MEDIA, march)
+    img, ms = {}, {}
+    for mode in (1, 7, 5):
+        g.set_option(pmamd.PM_OPT_GATHER_MODE, mode)
+        for _ in range(4):
+            img[mode] = g.render()
+            ms[mode] = min(ms.get(mode, 1e9), g.stats().ms_render)
+    say("ms: heap %.3f, packet %.3f, auto %.3f" % (ms[1], ms[7], ms[5]))
+    # the two differ by twice and more; the margin is for the clock
+    assert ms[5] < 1.4 * min(ms[1], ms[7]) + 0.02
+    assert np.array_equal(img[5], img[1]) or np.array_equal(img[5], img[7])
+    g.close()
+
+
+def test_default_of_a_sparse_batch_is_a_heap():
+    """A batch whose balls hold nothing is not given to the packet gather, the
+    batched workload's scenes are."""
+    say("case: default tuning of two batches")
+    for cap, mode in ((0.004, 0), (0.05, 7)):
+        cfgs = []
+        for i in range(3):
+            c = pmamd.batch_scene(5, i)
+            c.n_emit, c.width, c.height = 3000, 300, 280 + i
+            c.rcap_surface = c.rcap_volume = cap
+            c.medium, c.sigma_s, c.sigma_a = pmamd.PM_MEDIUM_HOMOGENEOUS, 0.1, 0.01
+            cfgs.append(c)
+        b = pmamd.Batch(cfgs)
+        assert b.stats().tuning.gather_mode == mode
+        b.submit()
+        imgs = [b.image(i) for i in range(3)]
+        b.set_tuning(32, 64, 64, 2, 7 - mode, 0)
+        b.submit()
+        for i in range(3):
+            np.testing.assert_allclose(b.image(i), imgs[i], rtol=RTOL, atol=0)
+
+
+def test_cache_values_of_sparse_maps():
+    """Auto gathers a cache frame's exact values with the heap where hardly any
+    record has a photon within the cap (the packet gather: 2.5 to 5 times its
+    time), and gives the same frame."""
+    say("case: cache frame, 640x360, r <= 0.003, every record gathered")
+    c = pmamd.preset(1)
+    c.n_emit, c.width, c.height = 3000, 640, 360
+    c.rcap_surface = c.rcap_volume = 0.003
+    g = pmamd.PhotonMapper(c)
+    g.emit()
+    g.build()
+    img, ms = {}, {}
+    for mode in (1, 7, 5):
+        g.cache_reset(1)
+        g.cache_configure(threshold=0.0, train_samples=1 << 14, batch=1 << 14)
+        g.set_option(pmamd.PM_OPT_GATHER_MODE, mode)
+        for _ in range(4):
+            img[mode] = g.render_cache()
+            ms[mode] = min(ms.get(mode, 1e9), g.cache_stats().ms_fallback)
+    say("ms of the exact values: heap %.3f, packet %.3f, auto %.3f" % (ms[1], ms[7], ms[5]))
+    assert ms[5] < 1.4 * min(ms[1], ms[7]) + 0.02
+    np.testing.assert_allclose(img[5], img[7], rtol=RTOL, atol=0)
+    g.close()
