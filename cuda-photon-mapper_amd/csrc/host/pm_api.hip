@@ -366,6 +366,7 @@ int pm_create(const pm_config* cfg, pm_context** out) {
   c->cfg = *cfg;
   memset(&c->stats, 0, sizeof(c->stats));
   hipError_t e = hipGetDevice(&c->device);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming);
@@ -429,9 +430,8 @@ int pm_build(pm_context* c) {
   HIPCHK(hipEventRecord(c->ev_join, c->stream2));
   HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
   HIPCHK(hipEventRecord(c->e1, c->stream));
-  // the render's work items: a tile has at least 4 pixels, or the launch is small
-  HIPCHK(c->items.ensure(4ull * packet_item_words((uint32_t)std::max<uint64_t>(
-                             (uint64_t)c->cfg.width * (uint64_t)c->cfg.height / 4u, 1u << 15))));
+  // the work items of the renders that use them, whatever size follows
+  HIPCHK(c->items.ensure(4ull * packet_item_words(packet_list_tiles(c->cus))));
   HIPCHK(hipStreamSynchronize(c->stream));
   c->stats.ms_build = elapsed_ms(c->e0, c->e1);
   c->built = true;
@@ -482,8 +482,7 @@ int render_crop_impl(pm_context* c, int x0, int y0, int w, int h, float* rgb_dev
   r.gather_mode = c->gather_mode;
   r.tile_regions = c->tile_regions;
   r.sample_lanes = c->sample_lanes;
-  r.cus = 256;
-  (void)hipDeviceGetAttribute(&r.cus, hipDeviceAttributeMultiprocessorCount, c->device);
+  r.cus = c->cus;
   if (counters) {
     r.counters = counters;
     HIPCHK(launch_fill_u32(reinterpret_cast<uint32_t*>(counters), 0u, 4, c->stream));
@@ -522,9 +521,6 @@ int render_crop_impl(pm_context* c, int x0, int y0, int w, int h, float* rgb_dev
     case 1: HIPCHK(launch_render_lane(r, c->stream)); break;
     case 4: HIPCHK(launch_render_lane4(r, c->stream)); break;
     case 7:
-      // the work items' scratch: grown here, or as pm_build left it for the
-      // caller that allocates nothing (a larger frame then renders in raster order)
-      if (!counters) HIPCHK(c->items.ensure(4ull * packet_item_words(packet_tiles(r))));
       r.items.head = c->items.as<uint32_t>();
       r.items.words = c->items.bytes / 4;
       HIPCHK(launch_render_packet(r, c->stream));

@@ -135,6 +135,7 @@ struct pm_context {
   int sample_lanes = 1;  // mode 7: a pixel's samples in adjacent lanes
   int render_media = 1;  // 0: the plain render gathers at surface hits only
   int voxel_grid = 0;    // 1: the plain render uses the voxel-grid estimate, 2: with the bilinear blend
+  int cus = 256;          // compute units of the device
   pm::DevBuf items;       // packet renders' work items
   bool vox_ready = false;  // voxel grids and tables hold the current records
   pm::DevBuf vox_grid_s, vox_grid_v, vox_sat_s, vox_sat_v;

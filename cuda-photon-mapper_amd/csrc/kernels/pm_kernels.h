@@ -163,6 +163,7 @@ struct RenderItems {
   uint32_t* light;  // tile
 };
 size_t packet_item_words(uint32_t tiles);
+uint32_t packet_list_tiles(int cus);  // more tiles than a launch with work items has
 struct RenderLaunch {
   Scene sc;
   RenderParams rp;
@@ -191,9 +192,8 @@ bool packet_pays(const RenderLaunch& r);
 bool packet_pays(const RenderParams& rp, bool march, const GatherMap& gs, const GatherMap& gv, int ls, int lu,
                  uint64_t pixels, int cus);
 bool packet_pays_rows(const GatherMap& gv);
-// Tiles of a packet render of r, and the lists of its heavy and light items
-// into r.items (head set, packet_item_words(tiles) words).
-uint32_t packet_tiles(const RenderLaunch& r);
+// The heavy and light items of a packet render of `tiles` tiles into r.items
+// (head set, packet_item_words(tiles) words).
 hipError_t launch_packet_tiles(RenderLaunch& r, int lu, int ls, uint32_t tiles, hipStream_t st);
 
 // voxel-grid compatibility mode (pm_voxel.hip): both maps splatted into

@@ -411,6 +411,9 @@ int packet_march_lanes_batch(const RenderParams& rp, const GatherMap& gv, uint64
 
 size_t packet_item_words(uint32_t tiles) { return 4 + 5ull * tiles; }
 
+// Launches of at least this many tiles take no work list (launch_render_packet).
+uint32_t packet_list_tiles(int cus) { return 64u * (uint32_t)cus; }
+
 // log2 of the samples of a pixel that go to adjacent lanes.
 static int packet_sample_lanes(const RenderLaunch& r) {
   const int spp = r.rp.spp;
@@ -493,11 +496,6 @@ bool packet_pays(const RenderLaunch& r) {
   return packet_pays(r.rp, r.rp.media_on != 0, r.gs, r.gv, ls, lu, (uint64_t)r.w * (uint64_t)r.h, r.cus);
 }
 
-uint32_t packet_tiles(const RenderLaunch& r) {
-  int lu, ls;
-  return packet_layout(r, lu, ls);
-}
-
 hipError_t launch_packet_tiles(RenderLaunch& r, int lu, int ls, uint32_t tiles, hipStream_t st) {
   r.items.heavy = r.items.head + 4;
   r.items.light = r.items.heavy + 4ull * tiles;
@@ -523,7 +521,7 @@ hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st) {
   // frame is to be the faster one there, and takes 10 to 11 ms.
   const double rm = mean_radius(r.gv);
   const bool dense = rm * rm < 0.999 * r.gv.rcap2;
-  const bool few = dense ? ls > 0 && tiles < 64u * (unsigned)r.cus : lu > 0 && tiles < 34u * (unsigned)r.cus;
+  const bool few = tiles < packet_list_tiles(r.cus) && (dense ? ls > 0 : lu > 0 && tiles < 34u * (unsigned)r.cus);
   if (r.tile_regions == 0 && r.rp.media_on && few && r.items.head && r.items.words >= packet_item_words(tiles)) {
     hipError_t e = launch_packet_tiles(q, lu, ls, tiles, st);
     if (e != hipSuccess) return e;

@@ -170,8 +170,9 @@ int pm_render_crop(pm_context* ctx, int x0, int y0, int w, int h, float* rgb_dev
 /* pm_render_crop without any allocation: no reference counterpart.  For
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops).  Same arguments, outputs and statistics as
- * pm_render_crop.  The render's only scratch, its two 64-bit query counters
- * (16 bytes), lives in a library-wide device array, one per GPU, held from
+ * pm_render_crop.  The render's scratch is the context's work list (0.3 MB,
+ * allocated by pm_build, for any frame size) and its two 64-bit query counters
+ * (16 bytes), which live in a library-wide device array, one per GPU, held from
  * library load to process end; the call clears it with a kernel before the
  * render.  Calls that overlap on one GPU (several host threads or contexts)
  * share that array and race on it.  The context must already be built (its

@@ -6,6 +6,7 @@ sum differs by at most its last bit between them, and a pixel's radiance (a
 sum of non-negative terms, each off by at most 2^-23 of itself, and the
 rounding of the sums) by less than 5e-7 of itself.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -204,4 +205,35 @@ def test_cache_values_of_sparse_maps():
     say("ms of the exact values: heap %.3f, packet %.3f, auto %.3f" % (ms[1], ms[7], ms[5]))
     assert ms[5] < 1.4 * min(ms[1], ms[7]) + 0.02
     np.testing.assert_allclose(img[5], img[7], rtol=RTOL, atol=0)
+    g.close()
+
+
+def free_device_bytes():
+    pmamd.load()
+    with open("/proc/self/maps") as f:  # the HIP runtime that libpm.so is linked to
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_work_list_memory_does_not_grow_with_the_frame():
+    """Only launches of fewer tiles than 64 a CU use the work list (0.3 MB), so
+    an 8192x8192 frame reserves no more for it: its build takes the trees of a
+    thousand photons and that list."""
+    say("case: device memory of a build, 8192x8192 frame")
+    c = pmamd.preset(1)
+    c.n_emit, c.width, c.height = 1000, 8192, 8192
+    g = pmamd.PhotonMapper(c)
+    g.emit()
+    before = free_device_bytes()
+    g.build()
+    assert before - free_device_bytes() < 64 << 20
+    # and a window of it renders from the list as ever
+    g.set_option(pmamd.PM_OPT_GATHER_MODE, 7)
+    a = g.render(4000, 4000, 64, 48)
+    before = free_device_bytes()
+    g.render(0, 0, 2048, 2048)
+    assert before - free_device_bytes() < (2048 * 2048 * 12) + (16 << 20)  # the caller's image
+    assert np.array_equal(a, g.render(4000, 4000, 64, 48))
     g.close()
