@@ -125,17 +125,40 @@ int sync_ema(pm_context* c) {
   return PM_OK;
 }
 
+// Space for the records of a frame of N; what was there (the seeds) is lost.
+int grow_records(CacheState& k, uint64_t N) {
+  const uint64_t n = (N + 127u) / 128u * 128u;  // every array starts on 256 bytes
+  k.rec_cap = k.rec_q_n = 0;
+  HIPCHK(k.rec.ensure(n * (4u * MLP_IN + 12u + 12u + 8u + 8u + 2u + 2u)));
+  char* p = (char*)k.rec.p;
+  auto take = [&](uint64_t bytes) {
+    char* a = p;
+    p += n * bytes;
+    return a;
+  };
+  k.rec_in = (float*)take(4u * MLP_IN);
+  k.rec_wt = (float*)take(12u);
+  k.rec_val = (float*)take(12u);
+  k.list = (uint32_t*)take(8u);
+  k.list_fb = (uint32_t*)take(8u);
+  k.rec_code = (uint16_t*)take(2u);
+  k.rec_q = (uint16_t*)take(2u);
+  k.rec_cap = n;
+  return PM_OK;
+}
+
 }  // namespace
 
 namespace pm {
 void cache_release(CacheState& k) {
   for (DevBuf* b : {&k.params, &k.grads, &k.adam_m, &k.adam_v, &k.params_bf16, &k.params_ema, &k.ema_bf16, &k.X, &k.y, &k.H[0], &k.H[1],
-                    &k.row_err, &k.rgb, &k.err_sum, &k.err_cnt, &k.rec_cnt, &k.rec_off, &k.rec_in,
-                    &k.rec_wt, &k.rec_code, &k.rec_val, &k.sel_in, &k.sel_t, &k.list, &k.list_cnt, &k.cell_fb,
-                    &k.row_code, &k.row_list, &k.loss_part, &k.loss_acc, &k.rec_q, &k.map_hash, &k.list_fb, &k.sel_order,
+                    &k.row_err, &k.rgb, &k.err_sum, &k.err_cnt, &k.rec_cnt, &k.rec_off, &k.rec,
+                    &k.sel_in, &k.sel_t, &k.list_cnt, &k.cell_fb,
+                    &k.row_code, &k.row_list, &k.loss_part, &k.loss_acc, &k.map_hash, &k.sel_order,
                     &k.XT, &k.dT[0], &k.dT[1], &k.dT[2], &k.dT[3], &k.dyT, &k.tpart})
     b->release();
   for (int l = 0; l < MLP_HIDDEN_LAYERS; ++l) k.HT[l].release();
+  k.rec_cap = k.rec_q_n = 0;
   k.ready = false;
 }
 
@@ -429,15 +452,15 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   }
   HIPCHK(hipStreamSynchronize(st));
   if (N >= 0xffffffffull) return PM_ERR_CAPACITY;
-  HIPCHK(k.rec_in.ensure(4ull * MLP_IN * std::max<uint64_t>(N, 1)));
-  HIPCHK(k.rec_wt.ensure(12ull * std::max<uint64_t>(N, 1)));
-  HIPCHK(k.rec_code.ensure(2ull * std::max<uint64_t>(N, 1)));
-  HIPCHK(k.rec_val.ensure(12ull * std::max<uint64_t>(N, 1)));
+  if (N > k.rec_cap || !k.rec.p) {
+    const int re = grow_records(k, std::max<uint64_t>(N, 1));
+    if (re != PM_OK) return re;
+  }
   rl.write = 1;
   rl.offsets = k.rec_off.as<uint32_t>();
-  rl.in = k.rec_in.as<float>();
-  rl.wt = k.rec_wt.as<float>();
-  rl.code = k.rec_code.as<uint16_t>();
+  rl.in = k.rec_in;
+  rl.wt = k.rec_wt;
+  rl.code = k.rec_code;
   HIPCHK(launch_cache_record(rl, st));
   HIPCHK(hipEventRecord(ev[1], st));
   // 4: online training on a subset with exact kNN targets
@@ -464,14 +487,13 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   auto prepare_seeds = [&]() -> int {
     if (seeds_checked || !mode7 || !k.use_seeds) return PM_OK;
     seeds_checked = true;
-    if (k.rec_q_n != N || !k.rec_q.p || hh[0] != k.rec_q_hash[0] || hh[1] != k.rec_q_hash[1]) {
-      HIPCHK(k.rec_q.ensure(2ull * std::max<uint64_t>(N, 1)));
-      HIPCHK(hipMemsetAsync(k.rec_q.p, 0xff, 2ull * N, st));
+    if (k.rec_q_n != N || hh[0] != k.rec_q_hash[0] || hh[1] != k.rec_q_hash[1]) {
+      HIPCHK(hipMemsetAsync(k.rec_q, 0xff, 2ull * N, st));
       k.rec_q_n = N;
       k.rec_q_hash[0] = hh[0];
       k.rec_q_hash[1] = hh[1];
     }
-    seeds = k.rec_q.as<uint16_t>();
+    seeds = k.rec_q;
     return PM_OK;
   };
   // when every surface record falls back (surfaces not cached), their exact
@@ -483,13 +505,12 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
     HIPCHK(k.sel_in.ensure(4ull * MLP_IN * S));
     HIPCHK(k.sel_t.ensure(12ull * S));
     // index lists of surface and volume records (in record order)
-    HIPCHK(k.list.ensure(8ull * std::max<uint64_t>(N, 1)));
     CacheListRule kinds;
     memset(&kinds, 0, sizeof(kinds));
     uint32_t nk[2] = {0, 0};
-    int rl_err = build_lists(c, k.rec_code.as<uint16_t>(), N, kinds, k.list.as<uint32_t>(), nk);
+    int rl_err = build_lists(c, k.rec_code, N, kinds, k.list, nk);
     if (rl_err != PM_OK) return rl_err;
-    const uint32_t* list_s = k.list.as<uint32_t>();
+    const uint32_t* list_s = k.list;
     const uint32_t* list_v = list_s + nk[0];
     if (!k.cache_surface) {
       infer_list = list_v;
@@ -503,10 +524,10 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
       CacheValueLaunch vs;
       memset(&vs, 0, sizeof(vs));
       vs.gs = gs; vs.gv = gv; vs.hg_g = c->scene.med.g;
-      vs.in = k.rec_in.as<float>();
+      vs.in = k.rec_in;
       vs.list = list_s;
       vs.n = nk[0];
-      vs.out = k.rec_val.as<float>();
+      vs.out = k.rec_val;
       vs.out_by_list = 1;
       vs.mode7 = mode7;
       vs.kind = 1;
@@ -518,7 +539,7 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
     // without surface caching the subset is drawn from the volume records only
     const uint32_t ns_sel = k.cache_surface ? nk[0] : 0u;
     if (ns_sel > 0 || nk[1] > 0) {  // else there is nothing the network answers, and nothing to train on
-      HIPCHK(launch_cache_select(k.rec_in.as<float>(), list_s, ns_sel, list_v, nk[1], S, c->cfg.seed, k.frame,
+      HIPCHK(launch_cache_select(k.rec_in, list_s, ns_sel, list_v, nk[1], S, c->cfg.seed, k.frame,
                                  k.sel_in.as<float>(), st));
       CacheValueLaunch vl;
       memset(&vl, 0, sizeof(vl));
@@ -542,13 +563,12 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   }
   HIPCHK(hipEventRecord(ev[2], st));
   // 5: inference over the records the cache may answer
-  int r = cache_predict_dev(c, k.rec_in.as<float>(), (uint32_t)N, k.rec_val.as<float>(), infer_list, n_infer);
+  int r = cache_predict_dev(c, k.rec_in, (uint32_t)N, k.rec_val, infer_list, n_infer);
   if (r != PM_OK) return r;
   HIPCHK(hipEventRecord(ev[3], st));
   // 6: exact fallback where the cache's cell error is high.  The list holds
   // the surface records, then the volume records, each in record order: a
   // wave then runs one kind of gather
-  HIPCHK(k.list.ensure(8ull * std::max<uint64_t>(N, 1)));
   HIPCHK(k.cell_fb.ensure(CACHE_CELLS));
   HIPCHK(launch_cache_cell_fb(k.err_sum.as<unsigned long long>(), k.err_cnt.as<unsigned int>(), k.threshold,
                               k.cell_fb.as<uint8_t>(), st));
@@ -557,8 +577,7 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
   fbr.cache_surface = k.cache_surface;
   fbr.cell_fb = k.cell_fb.as<uint8_t>();
   uint32_t nk2[2] = {0, 0};
-  HIPCHK(k.list_fb.ensure(8ull * std::max<uint64_t>(N, 1)));
-  r = build_lists(c, k.rec_code.as<uint16_t>(), N, fbr, k.list_fb.as<uint32_t>(), nk2);
+  r = build_lists(c, k.rec_code, N, fbr, k.list_fb, nk2);
   if (r != PM_OK) return r;
   const uint32_t nfb = nk2[0] + nk2[1];
   if (mode7 && nfb > 0) {
@@ -570,23 +589,23 @@ int pm_render_cache_crop(pm_context* c, int x0, int y0, int w, int h, float* rgb
     CacheValueLaunch vl;
     memset(&vl, 0, sizeof(vl));
     vl.gs = gs; vl.gv = gv; vl.hg_g = c->scene.med.g;
-    vl.in = k.rec_in.as<float>();
-    vl.list = k.list_fb.as<uint32_t>() + (kind == 2 ? nk2[0] : 0u);
+    vl.in = k.rec_in;
+    vl.list = k.list_fb + (kind == 2 ? nk2[0] : 0u);
     vl.n = nk2[kind - 1];
-    vl.out = k.rec_val.as<float>();
+    vl.out = k.rec_val;
     vl.out_by_list = 1;
     vl.mode7 = mode7;
     vl.kind = kind;
     vl.seed_q = seeds;
     if (mode7 && kind == 2)
-      HIPCHK(launch_order_rows(vl.in, k.list_fb.as<uint32_t>() + nk2[0], nk2[1], st));
+      HIPCHK(launch_order_rows(vl.in, k.list_fb + nk2[0], nk2[1], st));
     HIPCHK(launch_cache_values(vl, st));
   }
   if (surface_early) HIPCHK(hipStreamWaitEvent(st, c->ev_join, 0));
   HIPCHK(hipEventRecord(ev[4], st));
   // 7: per-pixel accumulation
-  HIPCHK(launch_cache_accumulate(k.rec_off.as<uint32_t>(), k.rec_cnt.as<uint32_t>(), w, h, k.rec_wt.as<float>(),
-                                 k.rec_val.as<float>(), c->rp.spp, c->cfg.exposure, rgb_dev, (uchar4*)out_dev, st));
+  HIPCHK(launch_cache_accumulate(k.rec_off.as<uint32_t>(), k.rec_cnt.as<uint32_t>(), w, h, k.rec_wt,
+                                 k.rec_val, c->rp.spp, c->cfg.exposure, rgb_dev, (uchar4*)out_dev, st));
   HIPCHK(hipEventRecord(ev[5], st));
   HIPCHK(hipStreamSynchronize(st));
   if (loss_terms) {

@@ -515,13 +515,15 @@ hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st) {
   dim3 grid(tile_grid(r, pk_tile_w(lp), pk_tile_h(lp), ls > 0));
   // The heavy tiles first and split where the launch ends on them: frames of
   // few waves, or, in a map so dense that a wave's march takes milliseconds, of
-  // few rounds of waves (480x270 window of the fog with 4 samples 30 -> 14 ms;
-  // the whole 1920x1080 frame 136 -> 151, so not there).  One-sample frames of
-  // such a map stay on the grid (the window: 23 ms, 11 from the list): a cache
-  // frame is to be the faster one there, and takes 10 to 11 ms.
+  // few rounds of waves.  Windows of the fog at the frame's centre, list
+  // against grid: 480x270 10.4 and 23.5 ms at 1 sample, 30 and 69 at 3, 21 and 35
+  // at 4; 1200x675 at 1: 30 and 74; the whole 1920x1080 frame at 4: 151 and 136,
+  // so not there.  With less than a tile a CU all waves start at once and the
+  // list only costs (120x68 at 1: 2.5 and 2.25).
   const double rm = mean_radius(r.gv);
   const bool dense = rm * rm < 0.999 * r.gv.rcap2;
-  const bool few = tiles < packet_list_tiles(r.cus) && (dense ? ls > 0 : lu > 0 && tiles < 34u * (unsigned)r.cus);
+  const bool few = dense ? tiles > (unsigned)r.cus && tiles < packet_list_tiles(r.cus)
+                         : lu > 0 && tiles < 34u * (unsigned)r.cus;
   if (r.tile_regions == 0 && r.rp.media_on && few && r.items.head && r.items.words >= packet_item_words(tiles)) {
     hipError_t e = launch_packet_tiles(q, lu, ls, tiles, st);
     if (e != hipSuccess) return e;

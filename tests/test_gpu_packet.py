@@ -237,3 +237,45 @@ def test_work_list_memory_does_not_grow_with_the_frame():
     assert before - free_device_bytes() < (2048 * 2048 * 12) + (16 << 20)  # the caller's image
     assert np.array_equal(a, g.render(4000, 4000, 64, 48))
     g.close()
+
+
+def test_dense_windows_end_on_split_tiles():
+    """Around the light of the fog scene a window of one sample a pixel is done
+    in less time than one of four, and three in a lane's loop in less than twice
+    theirs: without the heavy tiles first and in quarters, 1.1 and 3.3 times."""
+    say("case: 480x270 window of the fog at 1, 3 and 4 samples")
+    c = pmamd.preset(2)
+    g = pmamd.PhotonMapper(c)
+    g.emit()
+    g.build()
+    ms = {}
+    for spp in (1, 3, 4):
+        g.set_render(c.width, c.height, spp, c.k_surface, c.k_volume, c.rcap_surface, c.rcap_volume)
+        for _ in range(3):
+            g.render(720, 405, 480, 270)
+            ms[spp] = min(ms.get(spp, 1e9), g.stats().ms_render)
+    say("ms: %s" % ms)
+    assert ms[1] < 0.75 * ms[4] and ms[3] < 2 * ms[4]
+    g.close()
+
+
+def test_cache_frames_of_growing_size():
+    """A cache frame is the same after a smaller and a larger frame as in a new
+    context: the records' buffers grow and keep nothing."""
+    say("case: cache frames of 1, 4 and 2 samples in one context and alone")
+    c = pmamd.preset(1)
+    c.n_emit, c.width, c.height = 20000, 96, 64
+    g = pmamd.PhotonMapper(c)
+    g.emit()
+    g.build()
+    for spp in (1, 4, 2):
+        imgs = []
+        for own in (g, pmamd.PhotonMapper(c)):
+            if own is not g:
+                own.emit()
+                own.build()
+            own.set_render(96, 64, spp, c.k_surface, c.k_volume, c.rcap_surface, c.rcap_volume)
+            own.cache_reset(1)
+            own.cache_configure(threshold=0.05, train_samples=1 << 14, batch=1 << 12)
+            imgs.append(own.render_cache())
+        np.testing.assert_allclose(imgs[0], imgs[1], rtol=RTOL, atol=0)
