@@ -594,18 +594,35 @@ int apply_tuning(pm_batch* b, const pm_batch_tuning& t, bool capture_graph) {
     b->grid = prev_grid;
     return err;
   };
-  if (t.gather_mode == 7 && !b->tpayload.p) {
-    // the tree-ordered payload of gather mode 7, allocated on first use
-    const size_t N = std::max<size_t>((size_t)b->S_tot + b->V_tot, 1);
-    if (b->tpayload.ensure((b->bf16 ? 16 : 32) * N) != hipSuccess) return restore(PM_ERR_NOMEM);
-    if (t.leaf_size == b->L && (r = setup_scene_maps(b)) != PM_OK) return restore(r);
-  }
+  const int prev_L = b->L;
   if (t.leaf_size != b->L && (r = setup_forest(b, t.leaf_size)) != PM_OK) return restore(r);
+  if (t.gather_mode == 7 && !b->tpayload.p) {
+    // the tree-ordered payload of gather mode 7, allocated on first use and
+    // after all that every tuning needs
+    const size_t N = std::max<size_t>((size_t)b->S_tot + b->V_tot, 1);
+    if (b->tpayload.ensure((b->bf16 ? 16 : 32) * N) != hipSuccess) {
+      (void)hipGetLastError();  // not the next launch's error
+      if (prev_L > 0 && prev_L != b->L && (r = setup_forest(b, prev_L)) != PM_OK) return restore(r);
+      return restore(PM_ERR_NOMEM);
+    }
+    if ((r = setup_scene_maps(b)) != PM_OK) return restore(r);
+  }
   if (!capture_graph) {
     release_graph(b);
     return PM_OK;
   }
   return capture(b);
+}
+
+pm_batch_tuning heap_tuning(const pm_batch* b) {
+  pm_batch_tuning t;
+  t.leaf_size = 32;
+  t.block_threads = 64;
+  t.heap_slots = b->kmax <= 32 ? 32 : 64;
+  t.heap_key_bytes = 2;
+  t.gather_mode = 0;
+  t.top_levels = 0;
+  return t;
 }
 
 // The packet gather where it pays for most of the batch's samples, else the
@@ -628,13 +645,11 @@ pm_batch_tuning default_tuning(const pm_batch* b) {
         packet_pays(rp, rp.media_on != 0, gs, gv, 0, batch_march_lanes(b, s), b->npix, b->cus);
     (pays ? packet : heap) += (double)c.width * (double)c.height * (double)c.spp;
   }
-  pm_batch_tuning t;
-  t.leaf_size = 32;
-  t.block_threads = 64;
-  t.gather_mode = packet >= heap ? 7 : 0;
-  t.heap_slots = t.gather_mode == 7 || b->kmax > 32 ? 64 : 32;
-  t.heap_key_bytes = 2;
-  t.top_levels = 0;
+  pm_batch_tuning t = heap_tuning(b);
+  if (packet >= heap) {
+    t.gather_mode = 7;
+    t.heap_slots = 64;
+  }
   return t;
 }
 
@@ -722,7 +737,11 @@ int pm_batch_create(const pm_config* cfgs, int n, pm_batch** out) {
   int r = setup_scenes(b);
   if (r == PM_OK) r = size_records(b);
   if (r == PM_OK) r = setup_render(b);
-  if (r == PM_OK) r = apply_tuning(b, default_tuning(b), true);
+  if (r == PM_OK) {
+    r = apply_tuning(b, default_tuning(b), true);
+    // no room for the packet gather's payload copy: a heap needs none
+    if (r == PM_ERR_NOMEM) r = apply_tuning(b, heap_tuning(b), true);
+  }
   if (r != PM_OK) {
     destroy(b);
     return r;

@@ -209,7 +209,7 @@ def test_cache_values_of_sparse_maps():
 
 
 def free_device_bytes():
-    pmamd.load()
+    pmamd.load().pm_device_free(None)  # the runtime is up
     with open("/proc/self/maps") as f:  # the HIP runtime that libpm.so is linked to
         hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
@@ -279,3 +279,36 @@ def test_cache_frames_of_growing_size():
             own.cache_configure(threshold=0.05, train_samples=1 << 14, batch=1 << 12)
             imgs.append(own.render_cache())
         np.testing.assert_allclose(imgs[0], imgs[1], rtol=RTOL, atol=0)
+
+
+def test_batch_that_fits_only_without_the_payload_copy():
+    """The packet gather's copy of the payloads (32 bytes a record) is what a
+    batch can do without: where it does not fit beside the rest, the batch starts
+    with a heap, renders, and refuses the packet gather without harm."""
+    cfgs = []
+    for i in range(16):
+        c = pmamd.batch_scene(5, i)
+        c.n_emit, c.width, c.height = 2000000, 64, 64
+        c.medium, c.sigma_s, c.sigma_a = pmamd.PM_MEDIUM_HOMOGENEOUS, 0.1, 0.01
+        cfgs.append(c)
+    before = free_device_bytes()
+    b = pmamd.Batch(cfgs)
+    used = before - free_device_bytes()
+    st = b.stats()
+    copy = 32 * (st.surface_records + st.volume_records)
+    say("case: batch of %.1f GB, payload copy %.1f GB" % (used / 2**30, copy / 2**30))
+    assert st.tuning.gather_mode == 7 and copy > 2 << 30
+    b.submit()
+    img = b.image(3)
+    b.close()
+    filler = pmamd.DeviceBuffer(free_device_bytes() - used + copy // 2)
+    try:
+        b = pmamd.Batch(cfgs)
+        assert b.stats().tuning.gather_mode == 0
+        with pytest.raises(pmamd.PmError):
+            b.set_tuning(32, 64, 64, 2, 7, 0)
+        b.submit()
+        np.testing.assert_allclose(b.image(3), img, rtol=RTOL, atol=0)
+        b.close()
+    finally:
+        filler.free()
