@@ -65,7 +65,9 @@ __device__ __forceinline__ V3f psum_get(const PowerSum& s) { return v3((float)s.
 // |g| < 1 gives den >= 2^-48 for directions of unit length.  A longer one (BF16
 // storage rounds each component to 2^-9, and callers give their own) can take
 // den below 0: such a photon has no weight, as in phase_hg, whose Newton steps
-// underflow there (down to -0.2).
+// underflow there (down to -0.2; below that, and for infinite directions, they
+// give NaN, which a branch to them would keep at 3.7 % of the fog frame against
+// 1.2 for the select).
 struct HgPhase {
   float a, b, c;  // 1 + g^2, -2 g, (1 - g^2) / (4 pi)
 };
