@@ -10,7 +10,7 @@
 //           points within the bound of the query box are packed into LDS;
 //   count   every lane runs over the staged points (the same point for all
 //           lanes, one LDS broadcast) and counts them in a window of 128
-//           buckets of d^2 (FP32 bits >> 16, 2^-6 wide) around its previous
+//           buckets of d^2 (FP32 bits >> 16, 2^-7 wide) around its previous
 //           query's k-th-neighbour bucket, in 4-bit LDS counters; the bucket
 //           Q of its k-th neighbour is where the running count reaches k.  A
 //           lane whose k-th neighbour lies outside its window moves the
@@ -20,8 +20,10 @@
 //           all lanes; of the bucket-Q points the (d^2, index) smallest that
 //           complete k are picked at the end.
 // Queries that are not near each other are gathered in groups, each with its
-// own stage, so any set of queries gives the same neighbour sets; sums are in
-// FP64 (pm_estimate.h) and do not depend on the grouping.
+// own stage, so any set of queries gives the same neighbour sets.  The order
+// of their FP64 sums depends on the grouping, their FP32 results therefore in
+// the last bit now and then (pm_estimate.h): so do a crop and its frame, a batch
+// and a single scene, and seeded and unseeded rows.
 //
 // Bounds are exact: with the operation order of dist2 and monotonic FP32
 // rounding, no point has a smaller computed d^2 to a query than the computed

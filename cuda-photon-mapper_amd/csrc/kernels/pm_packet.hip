@@ -79,8 +79,8 @@ __device__ __forceinline__ V3f pk_scale(const GatherMap& g) { return v3(g.scale[
 // Eye sample s of pixel (px, py) for each lane with act set; every lane of
 // the wave calls it.  A sample has 2^lu adjacent lanes, all with its path; at
 // each turn of the march lane u of them takes step j0 + u, and the steps'
-// terms are then added in step order by all of them, so the sums are those of
-// one lane marching alone.
+// terms are then added in step order by all of them, as by one lane marching
+// alone.
 template <bool FP64T, bool CONE>
 __device__ __forceinline__ V3f packet_sample(const Scene& sc, const RenderParams& rp, const GatherMap& gs,
                                              const GatherMap& gv, PacketLds& S, int lane, int lu, bool act,
@@ -268,7 +268,7 @@ __device__ __forceinline__ void item_pixel(int lane, int lu, int ls, int lv, int
 // dielectric spread afterwards, and close to the light the neighbour balls
 // are small, so such a tile's queries fall into many groups and its wave takes
 // several times the others' time: it is listed first, in quarters of four
-// times the march lanes (the same pixels, bit for bit).
+// times the march lanes (the same queries, the steps' terms in the same order).
 constexpr float kNearLight = 0.1f;
 __device__ __forceinline__ bool heavy_ray(const Scene& sc, const RenderParams& rp, uint32_t px, uint32_t py, uint32_t s) {
   V3f o, d;

@@ -184,7 +184,11 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
                   float rcap_surface, float rcap_volume);
 
 /* Options.  PM_OPT_RENDER_MEDIA and PM_OPT_VOXEL_GRID change what is
- * estimated; the others change only how the GPU runs it, never the results:
+ * estimated; the others change only how the GPU runs it, never the neighbour
+ * sets.  Under the packet gather (mode 7) the order in which a query's
+ * neighbours are summed, in FP64, depends on how queries are grouped: between
+ * gather modes, a crop and its frame, and the options marked (*), the last bit
+ * of a radiance sum can differ (fewer than one sum in four million does):
  * PM_OPT_GATHER_MODE   0 = one wave64 per radiance query (cross-lane sorted list),
  *                      1 = one lane per query, 8x8 pixel tile per wave,
  *                          8-byte (d^2, index) heap keys in LDS,
@@ -208,7 +212,7 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                          buckets of d^2 (2^-7 wide) around the bucket of
  *                          its previous march step, then summed up to it;
  *                      (3 and 6 are not used: PM_ERR_INVALID);
- *                      every mode gives the same neighbour sets and images;
+ *                      every mode gives the same neighbour sets (*);
  * PM_OPT_BLOCKS_PER_CU workgroups per compute unit of the persistent mode-0 grid;
  * PM_OPT_CACHE_FUSED_INFER 4 = cache inference through one fused kernel, all
  *                      five layers with the activations in registers and the
@@ -226,11 +230,13 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                      0 = raster order (default), rx = 1, 2, 4 or 8 = the
  *                      frame cut into rx x (8 / rx) regions, one per XCD
  *                      (workgroups go to the 8 XCDs round-robin), so that each
- *                      XCD's L2 serves one compact part of the frame;
+ *                      XCD's L2 serves one compact part of the frame; regions
+ *                      take no work list, so a frame that would split its heavy
+ *                      tiles (*);
  * PM_OPT_SAMPLE_LANES  gather mode 7 with spp = 2, 4, 8 or 16: 1 = the samples of a
  *                      pixel in adjacent lanes (default; raster tile order),
  *                      0 = the wave loops over its pixels' samples
- *                      (PM_OPT_TILE_REGIONS applies to this form);
+ *                      (PM_OPT_TILE_REGIONS applies to this form) (*);
  * PM_OPT_RENDER_MEDIA  1 = pm_render / pm_render_crop / pm_render_cache_crop
  *                      march the medium (default, when the scene has one),
  *                      0 = they gather at surface hits only: the surface-gather
@@ -249,7 +255,7 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                      and auto) starts each record from its k-th neighbour's
  *                      bucket of the previous call while the records and the
  *                      photon positions are unchanged (default), 0 = unseeded
- *                      searches every call; the values are the same bits;
+ *                      searches every call (*);
  * PM_OPT_TOP_LEVELS    0..7, default 0: accepted, without effect (the packet
  *                      gather of mode 7 reads 64 nodes a step, so that no
  *                      top of the tree needs to be kept in LDS);
@@ -339,7 +345,7 @@ typedef struct pm_cache_stats {
  * the threshold, accumulate.  Same outputs as pm_render_crop.  While the
  * records and the photon positions stay the same from one call to the next,
  * the exact re-gathers start from each record's k-th-neighbour bucket of the
- * previous call (PM_OPT_CACHE_SEEDS; the same values, fewer passes). */
+ * previous call (PM_OPT_CACHE_SEEDS; the same neighbours, fewer passes). */
 int pm_render_cache_crop(pm_context* ctx, int x0, int y0, int w, int h, float* rgb_dev, pm_uchar4* out_dev);
 int pm_cache_stats_get(pm_context* ctx, pm_cache_stats* out);
 
@@ -348,11 +354,12 @@ int pm_cache_stats_get(pm_context* ctx, pm_cache_stats* out);
  * per frame by one hipGraph launch: batched emission over all scenes (one
  * count pass, one scan, one write pass), one kd-tree forest build over every
  * photon map, and one persistent render kernel fed by a device work queue of
- * (scene, 8x8 tile) items.  Every scene's records, trees and pixels are
- * bit-identical to its own pm_create/pm_emit/pm_build/pm_render run with the
- * same leaf size.  The workgroup size and heap slots never change a result;
- * the leaf size changes only the order in which the (identical) neighbours'
- * contributions are summed.  No reference counterpart (the reference renders
+ * (scene, tile) items.  Every scene's records and trees are bit-identical to its
+ * own pm_create/pm_emit/pm_build run with the same leaf size, and so are its
+ * pixels to pm_render's under the heap gather of the same keys; under the packet
+ * gather the last bit of a sum can differ (see the options above).  The workgroup
+ * size and heap slots never change a result; the leaf size changes only the
+ * order in which the (identical) neighbours' contributions are summed.  No reference counterpart (the reference renders
  * one scene). */
 typedef struct pm_batch pm_batch;
 
@@ -369,7 +376,7 @@ typedef struct pm_batch_tuning {
 
 typedef struct pm_batch_stats {
   uint32_t n_scenes;
-  uint32_t work_items;                       /* 8x8 tiles of all scenes */
+  uint32_t work_items;                       /* 8x8 tiles of all scenes (the packet gather's tiles can be smaller) */
   uint64_t photons, surface_records, volume_records, pixels;
   uint64_t surface_queries, volume_queries;  /* radiance queries of the last frame */
   double ms_frame;                           /* last pm_batch_submit: graph launch to completion */

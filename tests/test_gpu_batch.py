@@ -1,8 +1,8 @@
 """Batched scenes on the GPU: one hipGraph launch renders every scene.
 
 Bars:
-  * every scene's photon records, flux tally, kd-trees and image are
-    bit-identical to the same scene run alone (pm_create / pm_emit /
+  * every scene's photon records, flux tally and kd-trees are bit-identical to
+    the same scene run alone, and on these scenes the image is too (pm_create / pm_emit /
     pm_build / pm_render with the same leaf size);
   * workgroup size and heap slots never change a bit; another leaf size
     gives the same trees as the scene's own build with that leaf size and the

@@ -1,7 +1,8 @@
 """The packet gather (gather mode 7) at the sizes where its stages, windows,
 groups and tie handling change, on caller-given photon maps, against the
 8-byte heap gather (mode 1), which keeps exact (d^2, index) keys and shares
-none of that code.  Both sum a query's neighbours in FP64, so a query's FP32
+none of the search with it (both use the FP64 sums and the phase function).
+Both sum a query's neighbours in FP64, so a query's FP32
 sum differs by at most its last bit between them, and a pixel's radiance (a
 sum of non-negative terms, each off by at most 2^-23 of itself, and the
 rounding of the sums) by less than 5e-7 of itself.
