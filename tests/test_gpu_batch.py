@@ -2,8 +2,8 @@
 
 Bars:
   * every scene's photon records, flux tally and kd-trees are bit-identical to
-    the same scene run alone, and on these scenes the image is too (pm_create / pm_emit /
-    pm_build / pm_render with the same leaf size);
+    the same scene run alone, and on these scenes the image is too (pm_create /
+    pm_emit / pm_build / pm_render with the same leaf size);
   * workgroup size and heap slots never change a bit; another leaf size
     gives the same trees as the scene's own build with that leaf size and the
     same neighbour sets, summed in another order (agreement to 1e-5);
@@ -122,6 +122,7 @@ def assert_same_radiance(ref, img, bitwise, what):
                                     (16, 192, 64, 2, 0, 0), (32, 64, 64, 2, 7, 0), (8, 256, 64, 2, 7, 0),
                                     (32, 128, 64, 2, 7, 3), (16, 256, 64, 2, 7, 5), (32, 64, 64, 2, 7, 7)])
 def test_batch_tuning_invariance(batch, tuning):
+    # the last entry, top_levels, is accepted without effect
     cfgs, b = batch
     b.set_tuning(32, 64, 32, 2)
     b.submit()
