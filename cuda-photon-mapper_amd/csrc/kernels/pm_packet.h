@@ -37,13 +37,21 @@
 
 namespace pm {
 
-constexpr uint32_t kPkCand = 320;     // staged points
+// Sizes measured one at a time (render ms; "fog" the 1920x1080 frame with 4
+// samples, "window" its 480x270 crop around the light at 1 sample, "surfaces"
+// the frame without the march, "room" the 480x270 room, "batch" 8 scenes).
+constexpr uint32_t kPkCand = 320;     // staged points: what leaves 16 waves' LDS
 constexpr uint32_t kPkBuckets = 128;  // counting window (8 counters per LDS word)
-constexpr uint32_t kPkUp = 48;        // window top above the previous query's bucket
+// Window top above the previous query's bucket: lower ones stage fewer points
+// and move more windows.  16, 32, 48, 64: fog 156, 133.8, 129.4, 133.2.
+constexpr uint32_t kPkUp = 48;
 constexpr uint32_t kPkStack = 192;    // node stack (see pk_stage)
 constexpr uint32_t kPkTie = 8;        // bucket-Q points kept per lane
-constexpr uint32_t kPkSolo = 8;       // groups of at most this many queries: one query at a time
-constexpr uint32_t kPkSoloFew = 12;   // the same where at most 32 queries start
+// Groups of at most this many queries go one query at a time.  4, 8, 16: window
+// 11.3, 10.4, 10.2, surfaces 5.8, 5.6, 5.6, room 1.8, 2.0, 1.9, batch 19.0, 18.8,
+// 19.3.
+constexpr uint32_t kPkSolo = 8;
+constexpr uint32_t kPkSoloFew = 12;   // the same where at most 32 queries start (8 to 20: the same)
 constexpr uint32_t kPkNoSeed = 0xffffffffu, kPkFew = 0xfffffffeu;
 
 // LDS of one wave: 10 KB, 16 waves per CU.
@@ -299,7 +307,12 @@ __device__ __forceinline__ void packet_gather(const GatherMap& g, PacketLds& S, 
   }
   // Few queries at once (lists of rows far apart) use few lanes of the passes
   // below, so more of them go one at a time, and without seeds only the very
-  // near ones share a stage: 1.2M such rows of the fog map 4.5 -> 2.3 ms.
+  // near ones share a stage (1.2M such rows of the fog map 4.5 -> 2.3 ms).
+  // A group's half width in radii of its leader: without seeds 0.08, 0.15, 0.3:
+  // batch 17.7, 18.8, 22.0, the rest the same; else 0.5, 0.75, 1.0: surfaces 5.2,
+  // 5.6, 5.6, window 11.5, 10.4, 10.0, room 2.3, 2.0, 1.6, batch 20.7, 18.8, 18.2,
+  // 5M unseeded rows 107, 110, 113.  Halved where the stage is too small, down
+  // to the leader alone (from 0.01 or 0.1 of it: the same).
   const bool sparse = __builtin_popcountll(todo) <= 32;
   const uint32_t solo = sparse ? kPkSoloFew : kPkSolo;
   float shrink = 1.0f;
@@ -532,7 +545,7 @@ __device__ __forceinline__ void packet_gather(const GatherMap& g, PacketLds& S, 
         uint32_t pieces = 0u;
         M = pk_stage(g, S, lane, box, u2f(bound), [&](uint32_t m) {
           whole = false;
-          return rough && ++pieces > 4u ? false : count(m);
+          return rough && ++pieces > 4u ? false : count(m);  // 1, 4, 16: those rows 112.9, 110.1, 110.0
         });
         staged = whole ? bound : 0u;
         if (pieces > 4u) {

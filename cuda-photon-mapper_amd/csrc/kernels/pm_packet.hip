@@ -378,9 +378,11 @@ static double mean_radius(const GatherMap& gv) {
 // A frame's march lanes: as few as fill the chip with waves, while the steps of
 // a turn stay within a neighbour ball; of very few waves up to 16, since each
 // wave's chain of march turns is then all there is.  Room scene (r = 0.05) at
-// lu = 0, 1, 2, 3, 4: 64x48 pixels 1.47, 0.85, 0.54, 0.44, 0.37 ms; 256x256
-// 13.8, 6.0, 4.1, 3.1, 2.9 ms; 480x270 13.4, 6.9, 4.5, 3.6, 4.0 ms; fog
-// (r = 0.02) 1920x1080 with 4 samples in lanes at lu = 0, 1, 2: 159, 211, 356.
+// lu = 0, 1, 2, 3, 4: 64x48 pixels 12.4, 4.2, 1.7, 1.1, 0.7 ms; 256x256 7.4, 1.8,
+// 1.75, 1.5, 2.2 (rule: 3); 480x270 7.6, 1.9, 2.0, 2.3, 2.7 (2); 960x540 6.2, 3.7,
+// 3.3, 3.7, 6.4 (0: 28 waves a CU are too few there).  Fog (r = 0.02) at lu = 0,
+// 1, 2: 1920x1080 with 4 samples in lanes 146, 206, 349 from the list, with one
+// 48, 60, 96; 480x270 around the light with one 12.0, 10.4, 21.6 (1).
 int packet_march_lanes(const RenderParams& rp, const GatherMap& gv, int ls, uint64_t pixels, int cus) {
   if (!rp.media_on) return 0;
   int lu = 0;
@@ -398,9 +400,9 @@ int packet_march_lanes(const RenderParams& rp, const GatherMap& gv, int ls, uint
 // wave's queries longer along the rays and narrower across them, so the box
 // they span is smallest where the two balance: with pixel pitch p (at distance
 // 1) 8 p / sqrt(2^lu) against 2^lu march steps.  The constant was fitted to
-// render times (ms) at lu = 0, 1, 2, 3, k = 32, r <= 0.05, 10^6 photons a
-// scene: 128^2: 79, 36, 28, 27   256^2: 71, 39, 35, 39   512^2: 79, 53, 52, 69
-//   1024^2: 100, 73, 81, 117.
+// render times; 8 scenes at lu = 0, 1, 2, 3, k = 32, r <= 0.05, 250,000 photons
+// each (ms): 128^2: 21.9, 9.8, 5.7, 6.0   256^2: 24.1, 11.1, 9.1, 10.8   512^2:
+// 26.5, 17.9, 19.5, 27.6   1024^2: 46.4, 48.1, 58.1, 94.5; the rule takes 2, 2, 1, 1.
 int packet_march_lanes_batch(const RenderParams& rp, const GatherMap& gv, uint64_t pixels, int cus) {
   if (!rp.media_on) return 0;
   const double pitch = 1.0 / ((double)rp.focal * (double)rp.height);
@@ -516,9 +518,11 @@ hipError_t launch_render_packet(const RenderLaunch& r, hipStream_t st) {
   // The heavy tiles first and split where the launch ends on them: frames of
   // few waves, or, in a map so dense that a wave's march takes milliseconds, of
   // few rounds of waves.  Windows of the fog at the frame's centre, list
-  // against grid: 480x270 10.4 and 23.5 ms at 1 sample, 30 and 69 at 3, 21 and 35
-  // at 4; 1200x675 at 1: 30 and 74; the whole 1920x1080 frame at 4: 151 and 136,
-  // so not there.  With less than a tile a CU all waves start at once and the
+  // against grid: 480x270 10.3 and 21.9 ms at 1 sample, 30 and 69 at 3, 21 and 35
+  // at 4; 1200x675 at 1: 30 and 74; the whole 1920x1080 frame (129,600 tiles) at
+  // 4: 146 and 129, so not there (at 1 sample, 32,400 tiles, 48 and 59 still).
+  // Room (march lanes): 64x48 0.71 and 0.93, 256x256 1.55 and 1.98, 640x360 2.07
+  // and 3.34.  With less than a tile a CU all waves start at once and the
   // list only costs (120x68 at 1: 2.5 and 2.25).
   const double rm = mean_radius(r.gv);
   const bool dense = rm * rm < 0.999 * r.gv.rcap2;
@@ -610,10 +614,11 @@ int render_batch_packet_occupancy(int fp64, int cone, int block_threads) {
 constexpr uint32_t kRowNoSeed = 0xffffu, kRowFew = 0xfffeu;  // the 16-bit forms of kPkNoSeed and kPkFew
 
 // Rows per wave: 16 of the training rows and of volume lists of fewer than
-// 2^21, where the launch would hold few waves, since the waves whose rows are far apart, or near
-// the light, take several times the others' time and end the launch; 64, whose
-// lanes share more, in a longer list.  256,000 volume rows: 14.6 ms at 64, 4.6
-// at 16; 129M: 117 ms at 64, 204 at 16.
+// 2^21, where the launch would hold few waves, since the waves whose rows are
+// far apart, or near the light, take several times the others' time and end the
+// launch; 64, whose lanes share more, in a longer list.  256,000 volume rows:
+// 14.6 ms at 64, 4.6 at 16; 129M: 117 ms at 64, 204 at 16; the seeded fallback
+// of the 1920x1080 cache frame with the line at 2^18, 2^21, 2^24: 3.4, 3.5, 4.8.
 constexpr uint32_t kFewRows = 1u << 21;
 
 template <int KIND>
