@@ -10,9 +10,8 @@ the hit).  Inputs are synthetic (the scene is generated from Philox seed 1).
 Prints one JSON line.  `value` = radiance queries (surface + volume kNN
 density estimates) per second of whole-frame time.  `roofline` is for the
 dominant kernel (the render/gather kernel), with its duration measured by HIP
-events on the library's own stream inside libpm.so; it also carries the
-kernel's VALU issue rate from the committed counter profile, the roof it
-actually sits on.  `cpu_baseline` times the CPU oracle (same per-thread logic,
+events on the library's own stream inside libpm.so and its VALU instructions
+and HBM traffic from the committed counter profiles.  `cpu_baseline` times the CPU oracle (same per-thread logic,
 std::thread over the host-core share of one GPU) on a stratified sample of the
 same frame, and the 256x256 unit-room workload in full.  `cache_bf16` reports
 the frame in its BF16-power + learned-cache form (queries recorded, MLP
@@ -127,6 +126,7 @@ def run_surface_gather(g, cfg, steps):
                         "r<=%g, at the diffuse hits of the %dx%d x %d spp eye paths"
                         % (int(s.n_surface), cfg.k_surface, cfg.rcap_surface, cfg.width, cfg.height, cfg.spp),
             "ms_per_frame": round(t, 3), "surface_queries": q, "radiance_queries_per_s": round(q / (t * 1e-3), 1),
+            # k records a query, though neighbouring queries share them: a rate of use, not of traffic
             "bytes_per_query": bpq, "achieved_GBps": round(bpq * q / (t * 1e-3) / 1e9, 1),
             "frac_of_hbm_peak": round(bpq * q / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "control_uniform_walls": ctl}
@@ -327,16 +327,11 @@ def run_batch(steps, tune_stride, n_scenes=64, seed=1):
     # kernel, with events around its render (one launch, every scene's tiles)
     ms_emit, ms_build, ms_render = b.time_phases()
     log("batch phases, kernel by kernel: emit %.1f ms, build %.1f ms, render %.1f ms" % (ms_emit, ms_build, ms_render))
-    bf16 = cfgs[0].storage == pmamd.PM_STORE_BF16
-    ks = {c.k_surface for c in cfgs} | {c.k_volume for c in cfgs}
-    bpq = gather_bytes_per_query(max(ks), bf16)
-    achieved = bpq * q / (ms_render * 1e-3) / 1e9
-    tb = read_profile("traffic_batch_cfg4.json")
-    roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": (tb.get("bytes_per_launch") if tb else None),
-            "kernel": "k_render_batch (persistent work queue over every scene's tiles)",
-            "bytes_per_query": bpq, "queries_per_launch": int(q), "kernel_ms": round(ms_render, 3),
-            "phases_ms": {"emit": round(ms_emit, 3), "build": round(ms_build, 3), "render": round(ms_render, 3)}}
+    roof = gather_roofline("k_render_batch_packet (persistent work queue over every scene's tiles)"
+                           if best[4] == 7 else "k_render_batch (the same with the heap gather)",
+                           int(q), ms_render, *(("traffic_batch_cfg4.json", "valu_batch_cfg4.json")
+                                                if best[4] == 7 else (None, None)))
+    roof["phases_ms"] = {"emit": round(ms_emit, 3), "build": round(ms_build, 3), "render": round(ms_render, 3)}
     b.close()
     alone = 0.0
     # the one-scene gather with the same heap keys (or mode 7)
@@ -531,6 +526,33 @@ def read_profile(name):
 VALU_ISSUE_PEAK_PER_S = 256 * 4 * 2.4e9 / 4
 
 
+def gather_roofline(kernel, queries, kern_ms, traffic_file, valu_file):
+    """What a render launch keeps busy: its VALU wave instructions (counted once,
+    profiles/) over its live duration against the issue peak, and its HBM traffic
+    (counted likewise).  Queries share the points that they read, so bytes per
+    query times queries is no traffic and has no roof.  The counts hold for one
+    workload, told by its number of queries."""
+    vp = read_profile(valu_file) if valu_file else None
+    tr = read_profile(traffic_file) if traffic_file else None
+    vp = vp if vp and vp.get("queries_per_launch") == queries else None
+    tr = tr if tr and tr.get("queries_per_launch") == queries else None
+    s = kern_ms * 1e-3
+    roof = {"bound": "valu", "achieved": None, "peak": round(VALU_ISSUE_PEAK_PER_S / 1e9, 1),
+            "unit": "G wave instructions/s", "frac": None, "kernel": kernel, "queries_per_launch": queries,
+            "kernel_ms": round(kern_ms, 3), "traffic": None}
+    if vp:
+        roof["achieved"] = round(vp["sq_insts_valu"] / s / 1e9, 1)
+        roof["frac"] = round(vp["sq_insts_valu"] / s / VALU_ISSUE_PEAK_PER_S, 4)
+        roof["valu_insts_per_launch"] = vp["sq_insts_valu"]
+        roof["salu_insts_per_launch"] = vp.get("sq_insts_salu")
+        roof["source"] = "profiles/%s (rocprofv3 SQ_INSTS_VALU of the same kernel)" % valu_file
+    if tr:
+        roof["traffic"] = tr["bytes_per_launch"]
+        roof["hbm_GBps"] = round(tr["bytes_per_launch"] / s / 1e9, 1)
+        roof["hbm_frac"] = round(tr["bytes_per_launch"] / s / 1e9 / HBM_PEAK_GBS, 4)
+    return roof
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -539,7 +561,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=15.0)
     ap.add_argument("--gather-mode", type=int, default=5,
-                    help="0: wave per query; lane per query with 1: 8-byte, 2: 4-byte, 3/4/6/7: 2-byte heap keys; 5: auto")
+                    help="0: wave per query; lane per query with 1: 8-byte, 2: 4-byte, 4: 2-byte heap keys; 7: packet; 5: auto")
     ap.add_argument("--tile-regions", type=int, default=0,
                     help="0: raster tile order; 1, 2, 4, 8: per-XCD regions, that many across")
     ap.add_argument("--frame", type=str, default="", help="WxHxSPP override of the frame (profiling runs only)")
@@ -562,7 +584,7 @@ def main():
     ap.add_argument("--batch-steps", type=int, default=3, help="timed batch frames (0: skip the batch leg)")
     ap.add_argument("--batch-tune-stride", type=int, default=4)
     ap.add_argument("--top-levels", type=int, default=0,
-                    help="kd-tree levels the mode-7 render stages in LDS per wave (PM_OPT_TOP_LEVELS)")
+                    help="PM_OPT_TOP_LEVELS (accepted, without effect)")
     ap.add_argument("--voxel-steps", type=int, default=3,
                     help="timed frames of the voxel-grid compatibility mode (0: skip the leg)")
     ap.add_argument("--voxel-cpu-seconds", type=float, default=8.0)
@@ -589,22 +611,9 @@ def main():
     q_frame = stats.surface_queries + stats.volume_queries
     value = q_frame / sec_per_frame
     kern_ms = float(np.mean([p[3] for p in per]))
-    bpq = gather_bytes_per_query(cfg.k_volume, cfg.storage == pmamd.PM_STORE_BF16)
-    achieved = bpq * q_frame / (kern_ms * 1e-3) / 1e9
-    tr = read_profile("traffic_render_cfg2.json")
-    vp = read_profile("valu_render_cfg2.json")
-    roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": (tr.get("bytes_per_launch") if tr else None),
-            "kernel": "k_render_packet (eye ray + march + kNN gather, one search for a wave's queries)",
-            "bytes_per_query": bpq,
-            "queries_per_launch": int(q_frame), "kernel_ms": round(kern_ms, 3)}
-    if vp:
-        # the roof the kernel actually sits on: VALU instruction issue
-        roof["valu_issue"] = {"insts_per_launch": vp["sq_insts_valu"], "peak_insts_per_s": VALU_ISSUE_PEAK_PER_S,
-                              "frac": round(vp["sq_insts_valu"] / (kern_ms * 1e-3) / VALU_ISSUE_PEAK_PER_S, 4),
-                              "salu_insts_per_launch": vp.get("sq_insts_salu"),
-                              "source": "profiles/valu_render_cfg2.json (rocprofv3 SQ_INSTS_VALU of the same kernel)"}
+    roof = gather_roofline("k_render_packet (eye ray + march + kNN gather, one search for a wave's queries)",
+                           int(q_frame), kern_ms, *(("traffic_render_cfg2.json", "valu_render_cfg2.json")
+                                                    if args.gather_mode in (5, 7) else (None, None)))
     photons_traced = stats.n_emit_total
     emit_ms = float(np.mean([p[0] for p in per]))
     out = {
