@@ -186,25 +186,6 @@ PM_HD void camera_ray(const RenderParams& rp, uint32_t px, uint32_t py, uint32_t
   *o = v3<T>(T(rp.eye[0]), T(rp.eye[1]), T(rp.eye[2]));
 }
 
-// A gather type may answer volume queries one march step late (to merge the
-// exact second pass of step j with the first pass of step j + 1): it then
-// declares `static constexpr bool kDeferredVolume = true` and provides
-//   bool volume_defer(x, wo, w, c) -- queue this point; c = w * value of an
-//                                     earlier point when one is ready
-//   bool volume_flush(wo, c)       -- the last queued point's w * value (wo:
-//                                     the segment's view direction, which is
-//                                     also the queued point's)
-// The march adds the weighted values in step order either way, so the sum
-// is the same as with the immediate g.volume.
-template <class G, class = void>
-struct DeferredVolume {
-  static constexpr bool value = false;
-};
-template <class G>
-struct DeferredVolume<G, decltype((void)G::kDeferredVolume, void())> {
-  static constexpr bool value = G::kDeferredVolume;
-};
-
 // A gather type that only counts its queries (their number depends on the
 // path's geometry, never on its weights) declares
 // `static constexpr bool kCountOnly = true`: the march then skips the
@@ -260,17 +241,8 @@ PM_HD void march_segment(const Scene& sc, const RenderParams& rp, V3<T> o, V3<T>
       sampled = true;
     }
     V3<T> w = thr * (Tj * ds);
-    if constexpr (DeferredVolume<G>::value) {
-      V3<T> c;
-      if (g.volume_defer(x, wo, w, c)) nsum3_add(L, c);
-    } else {
-      V3<T> S = g.volume(x, wo, w);
-      nsum3_add(L, mul(w, S));
-    }
-  }
-  if constexpr (DeferredVolume<G>::value) {
-    V3<T> c;
-    if (g.volume_flush(wo, c)) nsum3_add(L, c);
+    V3<T> S = g.volume(x, wo, w);
+    nsum3_add(L, mul(w, S));
   }
   if constexpr (CountOnly<G>::value) return;
   T Tseg;

@@ -4,8 +4,9 @@
   pipeline must reproduce the plain render (1e-4 relative, as the plain
   parity bar): this pins recording, weights and accumulation.
 * The exact values of the training targets and the fallback come from
-  k_values (2-byte heap gather) under gather mode 3 and from k_values7 (the
-  gather of mode 7) under modes 7 and auto: cache frames must be the same bits.
+  k_values (2-byte heap gather) under gather modes 0 to 4 and from
+  k_values_packet under mode 7 (auto takes either): on this scene the cache
+  frames are the same bits.
 * After online training on the cache scene, the cache render must stay within
   3% (display RMSE) of the plain render on the same eye samples and add at
   most 15% to the plain render's error against a 64-spp plain render (the
@@ -176,7 +177,7 @@ def test_inference_rows(scene):
 
 
 def test_value_kernels_agree(scene):
-    say("case: cache frames with the exact values of gather mode 4 (k_values) and mode 7 (k_values7)")
+    say("case: cache frames with the exact values of gather mode 4 (k_values) and mode 7 (k_values_packet)")
     g = scene
     imgs, stats = [], []
     try:
