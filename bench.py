@@ -155,8 +155,7 @@ def run_wall_control(cfg, steps, bpq, n=1000000):
     g.set_records(pmamd.PM_MAP_SURFACE, pos, power, dirs, n)
     g.build()
     g.set_option(pmamd.PM_OPT_RENDER_MEDIA, 0)
-    # the measured leg's gather (mode 7): the automatic choice would pick the
-    # one-pass gather here, since this map alone holds fewer than 2^20 records
+    # the measured leg's gather (mode 7), whatever auto takes on this map
     g.set_option(pmamd.PM_OPT_GATHER_MODE, 7)
     npx = cfg.width * cfg.height
     rgb = pmamd.DeviceBuffer(npx * 12)

@@ -2,8 +2,8 @@
 //
 // Gather mode 2 (pm_lane_knn2.h) keeps FP32 d^2 keys: 16 KB of LDS per wave
 // at k = 64, 10 waves per compute unit.  Here the heap keeps a 16-bit,
-// order-preserving bucket of d^2 (its FP32 bits >> 15: exponent and the top 7
-// mantissa bits, i.e. buckets 2^-7 wide in relative d^2), 8 KB per wave, so
+// order-preserving bucket of d^2 (its FP32 bits >> 15: exponent and the top 8
+// mantissa bits, i.e. buckets 2^-8 wide in relative d^2), 8 KB per wave, so
 // the compute unit holds as many waves as its registers allow.
 //   pass 1: the k smallest buckets under the search bound; the largest, Q, is
 //           the bucket of the k-th neighbour;
@@ -12,7 +12,7 @@
 //           contribute.  The k-th of those
 //           gives the exact r_k.
 // The neighbour set is the exact (d^2, index)-ordered kNN set, as in modes 1
-// and 2.  A bucket holds the k-th neighbour and on average 1.5 k 2^-7 < 1
+// and 2.  A bucket holds the k-th neighbour and on average 1.5 k 2^-8 < 1
 // other point at k = 64, so the two kept keys nearly always suffice; when
 // more bucket points are needed, further exact passes pick them in order.
 #pragma once

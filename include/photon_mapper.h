@@ -194,7 +194,7 @@ int pm_set_render(pm_context* ctx, int width, int height, int spp, int k_surface
  *                          8-byte (d^2, index) heap keys in LDS,
  *                      2 = as 1 with 4-byte heap keys (d^2 only) and a second
  *                          fixed-radius pass for the exact neighbour set,
- *                      4 = as 2 with 2-byte keys (d^2 buckets 2^-7 wide),
+ *                      4 = as 2 with 2-byte keys (d^2 buckets 2^-8 wide),
  *                          the exact order restored inside the k-th bucket,
  *                          leaf points loaded 4 at a time under a
  *                          5-waves-per-SIMD register budget,
@@ -359,8 +359,8 @@ int pm_cache_stats_get(pm_context* ctx, pm_cache_stats* out);
  * pixels to pm_render's under the heap gather of the same keys; under the packet
  * gather the last bit of a sum can differ (see the options above).  The workgroup
  * size and heap slots never change a result; the leaf size changes only the
- * order in which the (identical) neighbours' contributions are summed.  No reference counterpart (the reference renders
- * one scene). */
+ * order in which the (identical) neighbours' contributions are summed.  No
+ * reference counterpart (the reference renders one scene). */
 typedef struct pm_batch pm_batch;
 
 typedef struct pm_batch_tuning {

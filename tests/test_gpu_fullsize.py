@@ -6,7 +6,8 @@
   of a few thousand queries bit-exact against the oracle's tree search; a
   64x64 crop of the 1920x1080 x 4 spp frame within 1e-4 relative per pixel.
 * The 64-scene batch (the generator's scenes at full size): every scene's
-  records, flux tally, trees and image bit-identical to the scene run alone
+  records, flux tally and trees bit-identical to the scene run alone, and on
+  these scenes its image too,
   with the same leaf size and gather, and the query counts add up.
 """
 import sys
