@@ -234,6 +234,16 @@ int batch_march_lanes(const pm_batch* b, int s) {
   return packet_march_lanes_batch(render_params(b->cfg[s]), gv, pixels, b->cus);
 }
 
+// An allocation that a smaller forest may not need.
+#define MEMCHK(expr)                                              \
+  do {                                                            \
+    hipError_t _e = (expr);                                       \
+    if (_e != hipSuccess) {                                       \
+      set_last_hip(_e, #expr);                                    \
+      return _e == hipErrorOutOfMemory ? PM_ERR_NOMEM : PM_ERR_HIP; \
+    }                                                             \
+  } while (0)
+
 // Forest tables for leaf size L, the per-scene gather maps, the build scratch.
 int setup_forest(pm_batch* b, int L) {
   const uint32_t nt = 2u * (uint32_t)b->ns;
@@ -287,25 +297,25 @@ int setup_forest(pm_batch* b, int L) {
   }
   const size_t N = (size_t)b->S_tot + b->V_tot;
   const size_t n1 = std::max<size_t>(nn, 1);
-  HIPCHK(b->nodes.ensure(sizeof(KdNode) * n1));
-  HIPCHK(b->nrange.ensure(sizeof(uint2) * n1));
+  MEMCHK(b->nodes.ensure(sizeof(KdNode) * n1));
+  MEMCHK(b->nrange.ensure(sizeof(uint2) * n1));
   DevBuf* tabs[6] = {&b->node_lo, &b->node_hi, &b->node_lc, &b->node_lb, &b->node_pbase, &b->level_nodes};
   const std::vector<uint32_t>* src[6] = {&nlo, &nhi, &nlc, &nlb, &npb, &lvl};
   for (int i = 0; i < 6; ++i) {
-    HIPCHK(tabs[i]->ensure(4 * n1));
+    MEMCHK(tabs[i]->ensure(4 * n1));
     if (!src[i]->empty())
       HIPCHK(hipMemcpy(tabs[i]->p, src[i]->data(), 4 * src[i]->size(), hipMemcpyHostToDevice));
   }
-  HIPCHK(b->node_child.ensure(8 * n1));
+  MEMCHK(b->node_child.ensure(8 * n1));
   if (nn) HIPCHK(hipMemcpy(b->node_child.p, nchild.data(), 8ull * nn, hipMemcpyHostToDevice));
-  HIPCHK(b->tree_root.ensure(4ull * nt));
-  HIPCHK(b->tree_pbase.ensure(4ull * nt));
+  MEMCHK(b->tree_root.ensure(4ull * nt));
+  MEMCHK(b->tree_pbase.ensure(4ull * nt));
   HIPCHK(hipMemcpy(b->tree_root.p, root.data(), 4ull * nt, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(b->tree_pbase.p, pbase.data(), 4ull * nt, hipMemcpyHostToDevice));
-  HIPCHK(b->point_tree.ensure(4 * std::max<size_t>(N, 1)));
+  MEMCHK(b->point_tree.ensure(4 * std::max<size_t>(N, 1)));
   for (uint32_t t = 0; t < nt; ++t)
     HIPCHK(launch_fill_u32(b->point_tree.as<uint32_t>() + b->tree_pbase_h[t], t, b->tree_n[t], b->stream));
-  HIPCHK(b->build_tmp.ensure(4 * kdforest_temp_words((uint32_t)N, nn)));
+  MEMCHK(b->build_tmp.ensure(4 * kdforest_temp_words((uint32_t)N, nn)));
   // node boxes (gather mode 7): 2 nl - 1 per tree, leaves and internal levels
   b->tree_desc.resize(nt);
   std::vector<uint32_t> lpref(nt + 1, 0u);
@@ -339,13 +349,13 @@ int setup_forest(pm_batch* b, int L) {
   }
   b->box_depth = bdepth;
   b->nleaves = lpref[nt];
-  HIPCHK(b->bmin.ensure(16ull * std::max<uint32_t>(nbox, 1)));
-  HIPCHK(b->bmax.ensure(16ull * std::max<uint32_t>(nbox, 1)));
-  HIPCHK(b->tree_desc_d.ensure(sizeof(KdTreeDesc) * nt));
+  MEMCHK(b->bmin.ensure(16ull * std::max<uint32_t>(nbox, 1)));
+  MEMCHK(b->bmax.ensure(16ull * std::max<uint32_t>(nbox, 1)));
+  MEMCHK(b->tree_desc_d.ensure(sizeof(KdTreeDesc) * nt));
   HIPCHK(hipMemcpy(b->tree_desc_d.p, b->tree_desc.data(), sizeof(KdTreeDesc) * nt, hipMemcpyHostToDevice));
-  HIPCHK(b->leaf_pref_d.ensure(4ull * (nt + 1)));
+  MEMCHK(b->leaf_pref_d.ensure(4ull * (nt + 1)));
   HIPCHK(hipMemcpy(b->leaf_pref_d.p, lpref.data(), 4ull * (nt + 1), hipMemcpyHostToDevice));
-  HIPCHK(b->level_pref_d.ensure(4ull * std::max<size_t>(lvpref.size(), 1)));
+  MEMCHK(b->level_pref_d.ensure(4ull * std::max<size_t>(lvpref.size(), 1)));
   if (!lvpref.empty())
     HIPCHK(hipMemcpy(b->level_pref_d.p, lvpref.data(), 4ull * lvpref.size(), hipMemcpyHostToDevice));
   HIPCHK(hipStreamSynchronize(b->stream));
@@ -566,6 +576,28 @@ int run_frame(pm_batch* b, double* ms) {
   return PM_OK;
 }
 
+// The forest of leaf size L in place of the present one.  The captured graph
+// goes first: it holds the present one's addresses and counts.  Without room
+// for the new forest the present one is set up again, or, if that fails too,
+// none is (b->L = 0).
+int change_forest(pm_batch* b, int L) {
+  const int prev = b->L;
+  release_graph(b);
+  const int r = setup_forest(b, L);
+  if (r == PM_OK) return r;
+  (void)hipGetLastError();  // not the next launch's error
+  b->L = 0;
+  if (prev > 0 && setup_forest(b, prev) != PM_OK) {
+    (void)hipGetLastError();
+    b->L = 0;
+  }
+  return r;
+}
+
+// Whether the forest is the tuning's: not after a change of leaf size that
+// could neither be made nor taken back for want of memory.
+bool forest_ready(const pm_batch* b) { return b->L == b->tune.leaf_size; }
+
 // capture_graph = false leaves the graph to the caller (the autotuner runs
 // the frame directly on the stream).
 int apply_tuning(pm_batch* b, const pm_batch_tuning& t, bool capture_graph) {
@@ -595,14 +627,14 @@ int apply_tuning(pm_batch* b, const pm_batch_tuning& t, bool capture_graph) {
     return err;
   };
   const int prev_L = b->L;
-  if (t.leaf_size != b->L && (r = setup_forest(b, t.leaf_size)) != PM_OK) return restore(r);
+  if (t.leaf_size != b->L && (r = change_forest(b, t.leaf_size)) != PM_OK) return restore(r);
   if (t.gather_mode == 7 && !b->tpayload.p) {
     // the tree-ordered payload of gather mode 7, allocated on first use and
     // after all that every tuning needs
     const size_t N = std::max<size_t>((size_t)b->S_tot + b->V_tot, 1);
     if (b->tpayload.ensure((b->bf16 ? 16 : 32) * N) != hipSuccess) {
       (void)hipGetLastError();  // not the next launch's error
-      if (prev_L > 0 && prev_L != b->L && (r = setup_forest(b, prev_L)) != PM_OK) return restore(r);
+      if (prev_L > 0 && prev_L != b->L) (void)change_forest(b, prev_L);
       return restore(PM_ERR_NOMEM);
     }
     if ((r = setup_scene_maps(b)) != PM_OK) return restore(r);
@@ -807,7 +839,8 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
   auto consider = [&](const pm_batch_tuning& t) -> int {
     if (t.heap_slots < b->kmax) return PM_OK;
     int r = apply_tuning(b, t, false);
-    if (r == PM_ERR_INVALID) return PM_OK;  // a candidate this device cannot run: skipped
+    // skipped: a candidate this device cannot run, or whose forest or payload copy does not fit
+    if (r == PM_ERR_INVALID || (r == PM_ERR_NOMEM && forest_ready(b))) return PM_OK;
     if (r != PM_OK) return r;
     double ms = 0.0, ms2 = 0.0;
     if ((r = trial(&ms)) != PM_OK) return r;
@@ -865,6 +898,7 @@ int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out,
 
 int pm_batch_submit(pm_batch* b) {
   if (!b) return PM_ERR_INVALID;
+  if (!forest_ready(b)) return PM_ERR_STATE;
   if (!b->exec) {
     int r = capture(b);
     if (r != PM_OK) return r;
@@ -892,6 +926,7 @@ int pm_batch_submit(pm_batch* b) {
 
 int pm_batch_time_phases(pm_batch* b, double* ms_emit, double* ms_build, double* ms_render) {
   if (!b || !ms_emit || !ms_build || !ms_render) return PM_ERR_INVALID;
+  if (!forest_ready(b)) return PM_ERR_STATE;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   struct EvGuard {
     hipEvent_t* e;
@@ -960,6 +995,7 @@ int pm_batch_get_records(pm_batch* b, int scene, int map, float* pos, float* pow
 int pm_batch_get_tree(pm_batch* b, int scene, int map, uint32_t* perm, float* split, uint32_t* axis, uint32_t n,
                       uint32_t ni) {
   if (!scene_ok(b, scene) || !perm) return PM_ERR_INVALID;
+  if (!forest_ready(b)) return PM_ERR_STATE;
   DevMap m = scene_map(b, scene, map);
   if (n != m.n || ni != (m.nl > 0 ? m.nl - 1 : 0)) return PM_ERR_INVALID;
   return tree_to_host(m, perm, split, axis);

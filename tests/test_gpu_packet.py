@@ -285,7 +285,8 @@ def test_cache_frames_of_growing_size():
 def test_batch_that_fits_only_without_the_payload_copy():
     """The packet gather's copy of the payloads (32 bytes a record) is what a
     batch can do without: where it does not fit beside the rest, the batch starts
-    with a heap, renders, and refuses the packet gather without harm."""
+    with a heap, renders, refuses the packet gather without harm, and the
+    autotuner chooses among the heaps."""
     cfgs = []
     for i in range(16):
         c = pmamd.batch_scene(5, i)
@@ -306,8 +307,21 @@ def test_batch_that_fits_only_without_the_payload_copy():
     try:
         b = pmamd.Batch(cfgs)
         assert b.stats().tuning.gather_mode == 0
+        # refused at the same and at another leaf size, whose forest fits
+        for leaf in (32, 16):
+            with pytest.raises(pmamd.PmError):
+                b.set_tuning(leaf, 64, 64, 2, 7, 0)
+            b.submit()
+            np.testing.assert_allclose(b.image(3), img, rtol=RTOL, atol=0)
+        best, _ = b.autotune(sample_stride=3)
+        assert best[4] == 0 and b.stats().tuning.gather_mode == 0
+        # a forest that does not fit: leaves of 2 give 47 million nodes of 48 bytes
+        b.set_tuning(32, 64, 64, 2, 0, 0)
+        rest = pmamd.DeviceBuffer(free_device_bytes() - (256 << 20))
         with pytest.raises(pmamd.PmError):
-            b.set_tuning(32, 64, 64, 2, 7, 0)
+            b.set_tuning(2, 64, 64, 2, 0, 0)
+        rest.free()
+        assert b.stats().tuning.leaf_size == 32
         b.submit()
         np.testing.assert_allclose(b.image(3), img, rtol=RTOL, atol=0)
         b.close()
