@@ -396,12 +396,15 @@ int pm_batch_scene_config(uint32_t seed, int index, pm_config* out);
  * Runs the sizing pass and captures the frame graph. */
 int pm_batch_create(const pm_config* cfgs, int n_scenes, pm_batch** out);
 int pm_batch_destroy(pm_batch* b);
+/* A tuning whose kd-tree forest or payload copy does not fit in device memory
+ * is refused (PM_ERR_NOMEM) and the former one stays. */
 int pm_batch_set_tuning(pm_batch* b, const pm_batch_tuning* t);
 /* Times the kd-build and a 1-in-`sample_stride` subset of the render work
  * items for a staged sweep: heap key width {8, 4, 2} x heap slots {32 (when
  * every k <= 32), 64} and gather mode 7, then leaf size {4, 8, 16, 32}, then
- * workgroup size {64, 128, 256}, each stage from the best so far; keeps the
- * fastest and returns it (and its time). */
+ * workgroup size {64, 128, 256}, each stage from the best so far; what does
+ * not fit in device memory is passed over; keeps the fastest and returns it
+ * (and its time). */
 int pm_batch_autotune(pm_batch* b, int sample_stride, pm_batch_tuning* best_out, double* best_ms_out);
 /* One frame of every scene (one graph launch); blocking. */
 int pm_batch_submit(pm_batch* b);
